@@ -100,7 +100,7 @@ struct sld_dev {
   double* fext0[3] = {};
   int32_t fext_func = -1;
   double* props = nullptr;
-  double* thresholds = nullptr;      // [nmat][4] Rf_AS, Rs_AS, Rf_SA, Rs_SA
+  double* law_const = nullptr;       // [nmat][8] sma::law_constants
   int32_t nmat = 0;
   double* rho = nullptr;
   int32_t* mat_of_elem = nullptr;
@@ -476,7 +476,7 @@ int enqueue_step(sld_dev* d, double dt, int scheme, double phi, int tn, KernelTi
     E.efor = d->efor;
     E.corner_slot = d->corner_slot;
     E.props = d->props;
-    E.thresholds = d->thresholds;
+    E.law_const = d->law_const;
     E.mat_of_elem = d->mat_of_elem;
     E.E_of_elem = d->E_of_elem;
     E.kg = d->kg;
@@ -858,9 +858,9 @@ int sld_dev_create(const sld_mesh_desc* mesh, const sld_material_desc* mat,
   d->nmat = mat->nmat;
   TRY(upload(&d->props, mat->props, (size_t)mat->nmat * 18, s)); track(d, d->props);
   {
-    std::vector<double> th((size_t)mat->nmat * 4);
-    for (int k = 0; k < mat->nmat; ++k) sma::mat_thresholds(mat->props + 18 * k, &th[4 * k]);
-    TRY(upload(&d->thresholds, th.data(), th.size(), s)); track(d, d->thresholds);
+    std::vector<double> lc((size_t)mat->nmat * 8);
+    for (int k = 0; k < mat->nmat; ++k) sma::law_constants(mat->props + 18 * (size_t)k, &lc[8 * (size_t)k]);
+    TRY(upload(&d->law_const, lc.data(), lc.size(), s)); track(d, d->law_const);
   }
   TRY(upload(&d->rho, mat->rho, (size_t)mat->nmat, s)); track(d, d->rho);
   std::vector<int32_t> me;

@@ -5,10 +5,10 @@
 //                 (mod_sld_solution_methods.f90:122-145 CD, :406-429 TW;
 //                 sld_updbcs.f90:79-114 + sld_funbou.f90:95-136); clears
 //                 f_int for the coloured scatter
-//   sld_element   SoA gather into LDS element tiles (relative coordinates
-//                 and displacements), reference Jacobian +
-//                 deformation gradient at the 8 Gauss points, SMA return
-//                 map, Kirchhoff stress, internal force
+//   sld_element   SoA gather, one node per lane (coordinates and
+//                 displacements relative to the element's first node),
+//                 reference Jacobian + deformation gradient at the 8 Gauss
+//                 points, SMA return map, Kirchhoff stress, internal force
 //                 (sld_element_operations.f90:119-256, elmca2.f90:105-111,
 //                 sld_elmpre.f90:149-162, sld_builtin_materials.f90:316-371,
 //                 sld_elmmat.f90:137-150, mod_matrix.f90:2327-2431).
@@ -64,21 +64,102 @@ __host__ __device__ __forceinline__ R hex_deriv(int a, int g, int k) {
   if (k == 1) return s * f[0] * f[2];
   return s * f[0] * f[1];
 }
-// Walsh-Hadamard form of the same derivatives.  With node signs s_am and GP
-// signs s_gm (bit m of the index: xi = 4, eta = 2, zeta = 1), c the GP
-// coordinate and (m1, m2) the two directions other than k,
-//   dN_a/dxi_k(g) = 1/8 s_ak (1 + c s_a1 s_g1)(1 + c s_a2 s_g2),
-// so sum_a x_a dN_a/dxi_k(g) = 1/8 [V(k) + c s_g1 V(k|m1) + c s_g2 V(k|m2)
-// + c^2 s_g1 s_g2 V(7)] with V(h) = sum_a (prod_{m in h} s_am) x_a, and
-// sum_g Q(g) dN_a/dxi_k(g) = 1/8 s_ak [U0 + c s_a1 U1 + c s_a2 U2
-// + c^2 s_a1 s_a2 U12] with U the sums over g of Q(g), s_g1 Q(g), s_g2 Q(g),
-// s_g1 s_g2 Q(g).  V and U are per element; only the signed weights differ
-// between lanes.
+// The same derivatives, direction by direction.  With node signs s_am, GP signs
+// s_gm and c the GP coordinate,
+//   dN_a/dxi_k(g) = s_ak / 2 * w(s_a1 s_g1) * w(s_a2 s_g2),
+// (m1, m2) the two directions other than k, w(+1) = (1 + c) / 2 and w(-1) =
+// (1 - c) / 2: a half difference along k and interpolations along m1 and m2.
+// An element's eight lanes hold one node and one Gauss point each, both with
+// the lane's sign bits, so each of the three combines the lane's own value with
+// that of one partner lane.  Lane l = 0..7 of an element has the sign bits
+// x = l2, y = l1 ^ l2, z = l0 ^ l2, which makes the partners across x, y and z
+// the lanes l ^ 7, l ^ 2 and l ^ 1: the three exchanges that are one DPP move
+// each (row_half_mirror and two quad permutations).
+//   Scales and signs are left out of the combinations: an interpolation is
+// v + r v', r = (1 - c) / (1 + c), and a difference v - v'.  The derivatives
+// they give are the true ones over HEX_SC = ((1 + c) / 2)^2 / 2, column k with
+// the factor s_gk.  Both cancel in H = G_u J^-1; the cofactors of the current
+// Jacobian carry HEX_SC^-2 and the product of the other two signs, and the
+// transposed combinations give back HEX_SC and, where column k of Q keeps the
+// factor s_gk, differences again: one constant, +-HEX_SC^3 by the product of
+// the lane's signs, stands for them all.
 constexpr double HEX_GPOS = 0.577350269189626;
-// node with sign bits (bx, by, bz) in the reference node order
-__host__ __device__ constexpr int hex_node(int bx, int by, int bz) {
-  return 4 * bz + (by ? 3 - bx : bx);
+constexpr double HEX_R = (1.0 - HEX_GPOS) / (1.0 + HEX_GPOS);
+constexpr double HEX_CP = 0.5 * (1.0 + HEX_GPOS);
+constexpr double HEX_SC = 0.5 * HEX_CP * HEX_CP;
+__device__ __forceinline__ int lane_bits(int l) { return l ^ (3 * ((l >> 2) & 1)); }   // 4 x + 2 y + z
+// reference node (-,-,-) (+,-,-) (+,+,-) (-,+,-) (-,-,+) ... of sign bits b;
+// the Gauss point of sign bits b is b itself (xi outer, zeta inner)
+__host__ __device__ constexpr int hex_node(int b) {
+  return 4 * (b & 1) + ((b & 2) ? 3 - ((b >> 2) & 1) : (b >> 2) & 1);
 }
+
+// The value v of the partner lane across direction DIR (0 = x, 1 = y, 2 = z).
+template <int DIR>
+__device__ __forceinline__ float partner(float v) {
+  constexpr int ctrl = DIR == 0 ? 0x141 : DIR == 1 ? 0x4E : 0xB1;
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), ctrl, 0xf, 0xf, true));
+}
+template <int DIR>
+__device__ __forceinline__ double partner(double v) {
+  constexpr int ctrl = DIR == 0 ? 0x141 : DIR == 1 ? 0x4E : 0xB1;
+  return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), ctrl, 0xf, 0xf, true),
+                          __builtin_amdgcn_mov_dpp(__double2loint(v), ctrl, 0xf, 0xf, true));
+}
+
+// v + r v' of a lane's own value and its partner's
+__device__ __forceinline__ float interp_of(float v, float w) { return __builtin_fmaf((float)HEX_R, w, v); }
+__device__ __forceinline__ double interp_of(double v, double w) { return __builtin_fma(HEX_R, w, v); }
+
+// Interpolation along DIR over (1 + c) / 2 (its transpose is the same
+// combination).  In FP32 the exchange folds into the sum.
+template <int DIR>
+__device__ __forceinline__ float interp(float v) {
+  return v + partner<DIR>((float)HEX_R * v);
+}
+template <int DIR>
+__device__ __forceinline__ double interp(double v) {
+  return __builtin_fma(HEX_R, partner<DIR>(v), v);
+}
+
+// Derivatives over HEX_SC, columns with their signs left out, of a nodal value:
+// the three share their first exchanges (6 in all).
+template <typename R>
+__device__ __forceinline__ void hex_grad(R x, R (&d)[3]) {
+  const R xz = partner<2>(x);
+  const R a = interp_of(x, xz), dz = x - xz;
+  const R ay = partner<1>(a);
+  const R b = interp_of(a, ay), dy = a - ay;
+  d[0] = b - partner<0>(b);
+  d[1] = interp<0>(dy);
+  d[2] = interp<0>(interp<1>(dz));
+}
+
+// The transpose: sum_g sum_k q_k(g) dN_a/dxi_k(g) over HEX_SC at the lane's
+// node, column k of q with the factor s_gk.
+template <typename R>
+__device__ __forceinline__ R hex_grad_t(R qx, R qy, R qz) {
+  const R b = qx - partner<0>(qx), c = interp<0>(qy), g = interp<1>(interp<0>(qz));
+  const R a = (b + c) + partner<1>((R)HEX_R * b - c);
+  return (a + g) + partner<2>((R)HEX_R * a - g);
+}
+
+// x less the value of the element's first lane (a broadcast within each half
+// of a 16-lane row)
+__device__ __forceinline__ double minus_first(double x) {
+  const long long v = __double_as_longlong(x);
+  long long t = __builtin_amdgcn_update_dpp(v, v, 0x150, 0xf, 0x3, false);   // row_newbcast:0
+  t = __builtin_amdgcn_update_dpp(t, v, 0x158, 0xf, 0xc, false);             // row_newbcast:8
+  return x - __longlong_as_double(t);
+}
+
+// The FP32 kernels form the same derivatives by Walsh-Hadamard sums: with V(h) = sum_a (prod_{m in h} s_am) x_a,
+//   sum_a x_a dN_a/dxi_k(g) = 1/8 [V(k) + c s_g1 V(k|m1) + c s_g2 V(k|m2)
+//   + c^2 s_g1 s_g2 V(7)],
+//   sum_g Q(g) dN_a/dxi_k(g) = 1/8 s_ak [U0 + c s_a1 U1 + c s_a2 U2
+//   + c^2 s_a1 s_a2 U12],
+// U the sums over g of Q(g), s_g1 Q(g), s_g2 Q(g), s_g1 s_g2 Q(g).  V and U are
+// per element and go through LDS.
 // in-place Walsh-Hadamard butterfly over bit m of an 8-slot array: slot
 // b | m becomes the signed difference (+ side minus - side)
 template <typename R>
@@ -685,7 +766,7 @@ struct ElemArgs {
   const double* coord[3];       // SoA reference coordinates
   const double* u[3];           // SoA displacement (ITER_K)
   const double* props;          // [nmat][18]
-  const double* thresholds;     // [nmat][4] mat_thresholds of each material
+  const double* law_const;      // [nmat][8] sma::law_constants of each material
   const int32_t* mat_of_elem;   // [nelem] or null
   const double* E_of_elem;      // [nelem] or null
   const double* kg;             // [nelem][2] bulk and shear modulus per element
@@ -763,22 +844,48 @@ __device__ inline sma::ReturnMap surrogate_or_exact(const ElemArgs& A, const sma
   return rm;
 }
 
-// Wave-level flag counters: one 64-bit atomic per wave and per set bit type.
+// Wave-level flag counters: 64-bit atomics on the wave's counter line, lane 0
+// adding its KF_AS count and lane 1 its KF_SA count in one instruction; the
+// other bits (rare) one by one.
 __device__ __forceinline__ void count_flags(unsigned long long* ctr, uint32_t fl, bool valid) {
-  if (__ballot(valid && fl != 0u) == 0ull) return;   // wave-uniform: nothing to count
+  if (!valid) fl = 0u;
+  if (__ballot(fl != 0u) == 0ull) return;   // wave-uniform: nothing to count
   ctr += 8 * (blockIdx.x % COUNTER_SLOTS);
-  const uint32_t bits[7] = {sma::FLAG_KF_AS, sma::FLAG_KF_SA, sma::FLAG_NEWTON_FAIL,
-                            sma::FLAG_EIGEN_FAIL, sma::FLAG_DETF_NONPOS,
-                            sma::FLAG_SURR_USED, sma::FLAG_SURR_FALLBACK};
+  static_assert(sma::FLAG_KF_AS == 1u && sma::FLAG_KF_SA == 2u, "counters 0 and 1");
   const int lane = threadIdx.x & 63;
+  const int n0 = __popcll(__ballot(fl & sma::FLAG_KF_AS));
+  const int n1 = __popcll(__ballot(fl & sma::FLAG_KF_SA));
+  const int n = lane == 0 ? n0 : n1;
+  if (lane < 2 && n) atomicAdd(ctr + lane, (unsigned long long)n);
+  const uint32_t bits[5] = {sma::FLAG_NEWTON_FAIL, sma::FLAG_EIGEN_FAIL, sma::FLAG_DETF_NONPOS,
+                            sma::FLAG_SURR_USED, sma::FLAG_SURR_FALLBACK};
+  if (__ballot(fl & (bits[0] | bits[1] | bits[2] | bits[3] | bits[4])) == 0ull) return;
 #pragma unroll
-  for (int b = 0; b < 7; ++b) {
-    unsigned long long m = __ballot(valid && (fl & bits[b]));
-    if (m && lane == 0) atomicAdd(ctr + b, (unsigned long long)__popcll(m));
+  for (int b = 0; b < 5; ++b) {
+    const unsigned long long m = __ballot(fl & bits[b]);
+    if (m && lane == 0) atomicAdd(ctr + 2 + b, (unsigned long long)__popcll(m));
   }
 }
 
+// Orders one wave's LDS accesses (an element's eight lanes sit in one wave,
+// whose LDS operations complete in order): no wait and no workgroup barrier.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // EPB elements per block, 8 threads (one per Gauss point) per element.
+// What bounds it: VALU issue, 75% of the cycles at ~2.05 GHz (C1, FP64: ~750
+// instructions a wave, 3 of 4 in FP64), the rest the first loads of a wave and
+// the launch's start and end.  In FP64 an element's lanes exchange values by
+// DPP moves (hex_grad, hex_grad_t) instead of through LDS: with Walsh-Hadamard
+// sums and Gauss-point rows in LDS (175 FP64 values read or written per lane)
+// the LDS of a CU, shared by its four SIMDs, was as busy as the VALU, and the
+// two overlapped poorly.  FP64 element launch, before -> with exchanges: C1
+// 400x20x20 46.7 -> 39.2 us; 631 000 elements in 64 specimens 191 -> 167;
+// 691 000 elements of SMA tube in tissue 159 -> 125; 2583 damped elements
+// 8.0 -> 6.5.
 // R = kinematics/stress precision; the return map is always FP64.
 // SUR = 0 plain; 1 surrogate prepass (flags + features of transforming
 // points, no stress, no scatter); 2 element step using accepted surrogate
@@ -797,13 +904,13 @@ __device__ __forceinline__ void count_flags(unsigned long long* ctr, uint32_t fl
 // LAWS = 0: each element takes its own law (law_of_elem); LAWS = 1: every
 // element of the launch is SMA (a mesh without neo-Hookean elements, or the
 // SMA range of a law-grouped mesh), without the neo-Hookean path, whose
-// registers would otherwise add to the SMA path's (FP64: 124 VGPRs and 4
-// waves per SIMD against 163 and 3); LAWS = 2: every element of the launch
+// registers would otherwise add to the SMA path's (FP64: 126 VGPRs and 4
+// waves per SIMD against 167 and 3); LAWS = 2: every element of the launch
 // is neo-Hookean (the tissue range of a law-grouped mesh), without the SMA
-// path (FP64: 128 VGPRs, 4 waves per SIMD, a few values spilled; it runs 5%
-// faster than at 3 waves without spills; FP32: 64 VGPRs, 8 waves, 4.3 KB of
-// LDS per workgroup).  Kernels that also store the stresses (STORE) keep 3
-// waves in FP64 and 6 in the FP32 neo-Hookean kernel, where more would spill.
+// path (FP64: 108 VGPRs; FP32: 56, 8 waves).  FP64 and FP32 SMA kernels at 5
+// waves per SIMD spill 10 registers and run slower (C1: 44.6 against 40.4 us
+// and 30.5 against 28.9).  Kernels that also store the stresses (STORE) keep 3
+// waves in FP64 and 6 in the FP32 neo-Hookean kernel.
 template <typename R, int LAWS = 0, bool DAMP = false, bool STORE = false>
 struct ElemOccupancy {
   static constexpr int waves = DAMP ? (sizeof(R) == 8 ? 1 : 2)
@@ -855,51 +962,40 @@ template <typename R, int EPB, bool STORE, int SUR = 0, bool GATHER = false, int
 __global__ void __launch_bounds__(EPB * 8, (ElemOccupancy<R, LAWS, DAMP, STORE>::waves))
     sld_element(ElemArgs A) {
   constexpr int NC = DAMP ? 9 : 6;        // gathered components: x, u (, v)
+  // Two forms of the element's sums.  FP64 (XCH): exchanges between the lanes
+  // (hex_grad, hex_grad_t).  FP32: Walsh-Hadamard sums through LDS, the
+  // arithmetic that mode's runs have had: a change of rounding in FP32 grows to
+  // 2e-4 of the velocities in 200 steps of a cantilever.  (With exchanges the
+  // FP32 element launch takes 27.8 instead of 30 us on C1.)
+  constexpr bool XCH = sizeof(R) == 8;
   constexpr int NQ = DAMP ? 15 : 9;
-  // The relative nodal values are dead once V(h) is formed (a barrier
-  // follows), before the Gauss-point rows are first written: one LDS block
-  // serves both (the barrier at the end of a tile keeps the next tile's
-  // gather off the rows phase 3 still reads).  Each element's block is
-  // padded (lds_block) so that the 8 elements of a wave start in different
-  // LDS banks: the eight lanes of an element read the same value at once,
+  // One LDS block per element (byte offsets; an element's eight lanes sit in
+  // one wave, so wave_sync orders them and no workgroup barrier is needed).
+  // XCH: the rows of j through the law (FP64), the material constants.  FP32:
+  // the relative nodal values, then the Gauss-point rows of Q; V(h), then
+  // (without damping) the U sums; the material constants.
+  // Blocks are padded (lds_block) so that the 8 elements of a wave start in
+  // different LDS banks: the eight lanes of an element read one value at once,
   // and unpadded power-of-two strides put all eight elements' values in one
-  // bank.
-  // The rows of the relative values and of the Gauss-point values have 9
-  // entries (18 banks apart in FP64), so that the 8 lanes of an element
-  // reading 8 different rows hit different banks, and FP64 U rows 5.
-  // Without damping, V(h) is dead once the kinematics are formed, and the U
-  // sums (and the FP64 det J kept through the law) take its block.
-  constexpr bool U4_IN_V = !DAMP;
-  constexpr int ROW = 9;
-  constexpr int U4S = (!DAMP && sizeof(R) == 8) ? 5 : 4;
-  constexpr int VC = DAMP ? 10 : ((LAWS == 2 || sizeof(R) == 8) ? 6 : 8);  // V(h) row
-  constexpr int U4R = DAMP ? 11 : 8;
-  constexpr int RELN = lds_block(NC * ROW, sizeof(R));
-  constexpr int QN = lds_block(NQ * ROW, sizeof(R));
-  constexpr int VN = lds_block(U4_IN_V ? (8 * VC > U4R * U4S ? 8 * VC : U4R * U4S) : 8 * VC,
-                               sizeof(R));
-  constexpr int UN = U4_IN_V ? 1 : lds_block(U4R * U4S, sizeof(R));
-  __shared__ union {
-    R rel[EPB][RELN];                     // [c][a]: x_a - x_0 (0..2), u_a - u_0 (3..5), v_a - v_0 (6..8)
-    R q[EPB][QN];                         // [j][g]: Q(3i+k) (, q_i, z_k) at each Gauss point
-  } s_relq;
-  // V(h) of the components ([h][c]; FP32 rows of 8 for aligned reads, FP64
-  // rows of 6 are 16-byte aligned already)
-  __shared__ R s_vm[EPB][VN];
-  __shared__ R s_u4m[U4_IN_V ? 1 : EPB][UN];  // [j][0..3]: U0, U1, U2, U12 of Q(0..7) (, z_0..2)
-  auto s_rel = [&](int l) { return reinterpret_cast<R(*)[ROW]>(&s_relq.rel[l][0]); };
-  auto s_q = [&](int l) { return reinterpret_cast<R(*)[ROW]>(&s_relq.q[l][0]); };
-  auto s_v = [&](int l) { return reinterpret_cast<R(*)[VC]>(&s_vm[l][0]); };
-  auto s_u4 = [&](int l) {
-    if constexpr (U4_IN_V) return reinterpret_cast<R(*)[U4S]>(&s_vm[l][0]);
-    else return reinterpret_cast<R(*)[U4S]>(&s_u4m[l][0]);
-  };
-  __shared__ R s_wq[DAMP ? EPB : 1][3][8];   // Walsh-Hadamard coefficients of q_i
-  __shared__ double s_v0[DAMP ? EPB : 1][3]; // node 0's velocity
+  // bank.  Rows of 9 let the lanes of an element that read different rows hit
+  // different banks.
+  constexpr bool JLDS = sizeof(R) == 8;
+  constexpr int ROW = 9, VC = DAMP ? 10 : LAWS == 2 ? 6 : 8, U4R = DAMP ? 11 : 8;
+  constexpr int V_OFF = XCH ? (JLDS ? 9 * 8 * 8 : 0) : (NQ * ROW * 4 + 15) / 16 * 16;
+  constexpr int U_OFF = !XCH && DAMP ? V_OFF + 8 * VC * 4 : V_OFF;
+  constexpr int W_OFF = U_OFF + (XCH ? 0 : DAMP ? U4R * 16 : 8 * VC * 4);   // damping: WHT of q_i
+  constexpr int C_OFF = W_OFF + (!XCH && DAMP ? 3 * 8 * 4 : 0);
+  constexpr int BLK = lds_block(C_OFF + 10 * 8, 1);
+  __shared__ __align__(16) unsigned char s_blk[EPB][BLK];
+  auto s_row = [&](int l) { return reinterpret_cast<double(*)[8]>(&s_blk[l][0]); };
+  auto s_q = [&](int l) { return reinterpret_cast<R(*)[ROW]>(&s_blk[l][0]); };
+  auto s_v = [&](int l) { return reinterpret_cast<R(*)[VC]>(&s_blk[l][V_OFF]); };
+  auto s_u4 = [&](int l) { return reinterpret_cast<R(*)[4]>(&s_blk[l][U_OFF]); };
+  auto s_wq = [&](int l) { return reinterpret_cast<R(*)[8]>(&s_blk[l][W_OFF]); };
+  auto s_c = [&](int l) { return reinterpret_cast<double*>(&s_blk[l][C_OFF]); };
+  __shared__ double s_v0[!XCH && DAMP ? EPB : 1][3];   // node 0's velocity
 
   if (A.health->halted) return;
-  const int tid = threadIdx.x;
-  const int le = tid >> 3, g = tid & 7;
   int bid = blockIdx.x;
   if (A.xcd_remap) {
     // workgroups are dealt round-robin to the 8 XCDs: workgroup b runs on
@@ -915,155 +1011,214 @@ __global__ void __launch_bounds__(EPB * 8, (ElemOccupancy<R, LAWS, DAMP, STORE>:
   const int per = A.tiles_per_block > 0 ? A.tiles_per_block : 1;
   const int t_begin = bid * per, t_end = min(ntiles, t_begin + per);
   for (int blk = t_begin; blk < t_end; ++blk) {
-  const int i_el = A.e_begin + blk * EPB + le;
-  const bool valid = i_el < A.e_end;
-  const int e = !valid ? 0 : A.elem_list ? A.elem_list[i_el] : i_el;
+  // the thread index passes through an empty asm in every phase, so that what
+  // is derived from it (LDS addresses, the element, signed weights) is formed
+  // again where it is used and not held in registers through the law
+  const int tid = opaque(threadIdx.x);
+  // element, and the lane's Gauss point (its sign bits) and corner
+  const int le = tid >> 3, lb = XCH ? lane_bits(tid & 7) : tid & 7;
+  const int corner = XCH ? hex_node(lb) : tid & 7;
+  // lanes beyond the range repeat the last element: they load and compute as
+  // the others do and only their stores and counts are left out
+  const int i0 = A.e_begin + blk * EPB;
+  const bool valid = i0 + le < A.e_end;
+  const int lel = min(le, A.e_end - 1 - i0);
+  const int e = (!GATHER && A.elem_list) ? A.elem_list[i0 + lel] : i0 + lel;
+  // entry k (Gauss point or corner) of the lane's element: the tile's first
+  // one, the same for all lanes, plus a 32-bit offset where the elements
+  // follow each other
+  auto at = [&](auto* ptr, int k) {
+    if constexpr (GATHER) return ptr + (int64_t)i0 * 8 + (unsigned)(lel * 8 + k);
+    else return ptr + ((int64_t)e * 8 + k);
+  };
   if constexpr (SUR == 1) {
     // prepass: a workgroup without a candidate element only marks its
     // points as not listed (workgroup-uniform, before any barrier)
     if (A.sur_cand && !__syncthreads_or(valid && A.sur_cand[e])) {
-      if (valid) A.sur_status[(int64_t)e * 8 + g] = 0;
+      if (valid) *at(A.sur_status, lb) = 0;
       continue;
     }
   }
 
-  // -- phase 1: gather the element's 8 nodes (thread g loads node g); node
-  // 0's values come from the element's first lane by a wave shuffle
-  int node = 0;
+  // -- phase 1: the lane's node.  All of the tile's loads are issued here, in
+  // the order of their use: the indices (connectivity, material, corner slot),
+  // the nodal values, one material constant per lane (the element's 8
+  // constants and 2 moduli go through LDS) and the point's history, so that a
+  // wave waits for memory twice and not at every use.
+  const int node = *at(A.lnods, corner);
+  const int mat = A.mat_of_elem ? A.mat_of_elem[e] : 0;
+  int slot = 0;
+  if constexpr (GATHER) slot = *at(A.corner_slot, corner);
   double xa[NC];
 #pragma unroll
-  for (int c = 0; c < NC; ++c) xa[c] = 0.0;
-  if (valid) {
-    node = A.lnods[(int64_t)e * 8 + g];
-    xa[0] = A.coord[0][node];
-    xa[1] = A.coord[1][node];
-    xa[2] = A.coord[2][node];
-    xa[3] = A.u[0][node];
-    xa[4] = A.u[1][node];
-    xa[5] = A.u[2][node];
-    if constexpr (DAMP) {
-      xa[6] = A.vel[0][node];
-      xa[7] = A.vel[1][node];
-      xa[8] = A.vel[2][node];
-    }
-  }
-  {
-    const int lane0 = (tid & 63) & ~7;   // lane of the element's node 0
+  for (int c = 0; c < 3; ++c) xa[c] = A.coord[c][node];
 #pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      const double x0 = __shfl(xa[c], lane0, 64);
-      if (valid) s_rel(le)[c][g] = (R)(xa[c] - x0);
-      if constexpr (DAMP)
-        if (c >= 6 && valid && g == 0) s_v0[le][c - 6] = x0;
-    }
+  for (int c = 0; c < 3; ++c) xa[3 + c] = A.u[c][node];
+  if constexpr (DAMP) {
+#pragma unroll
+    for (int c = 0; c < 3; ++c) xa[6 + c] = A.vel[c][node];
   }
-  __syncthreads();
-  // thread c: V(h) of component c, nodes taken in sign-bit order
-  if (valid && g < NC) {
-    for (int c = opaque(g); c < NC; c += 8) {
+  const bool neo = LAWS == 2 || (LAWS == 0 && A.law_of_elem && A.law_of_elem[e]);
+  // constant l of the element's material, and its bulk (even l) or shear modulus
+  const int l8 = tid & 7;
+  const double c8 = LAWS == 2 ? A.props[18 * (int64_t)mat + (l8 & 1)] : A.law_const[8 * (int64_t)mat + l8];
+  double c2 = 0.0;
+  if constexpr (LAWS != 2) c2 = A.kg[2 * (int64_t)e + (l8 & 1)];
+  // a neo-Hookean element has no history: its values stay as they are in
+  // both slots (equal from creation and every set), so they are neither
+  // read nor written
+  double xS0 = 0.0, FAS0 = 0.0, FSA0 = 0.0;
+  if (!neo) {
+    xS0 = *at(A.sdv_n[0], lb);
+    FAS0 = *at(A.sdv_n[1], lb);
+    FSA0 = *at(A.sdv_n[2], lb);
+  }
+  // nodal values relative to the element's first node (formed in FP64), so that
+  // coordinates far from the origin lose no more digits than one subtraction
+  R xr[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) xr[c] = (R)(c < 6 || !XCH ? minus_first(xa[c]) : xa[c]);
+  if constexpr (!XCH) {
+#pragma unroll
+    for (int c = 0; c < NC; ++c) s_q(le)[c][corner] = xr[c];
+    if constexpr (DAMP)
+      if (lb == 0) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) s_v0[le][c] = xa[6 + c];
+      }
+    wave_sync();
+    // lane c: V(h) of component c
+    const int t1 = opaque(tid), l1 = t1 >> 3;
+    for (int c = t1 & 7; c < NC; c += 8) {
       R v[8];
 #pragma unroll
-      for (int b = 0; b < 8; ++b) v[b] = s_rel(le)[c][hex_node((b >> 2) & 1, (b >> 1) & 1, b & 1)];
+      for (int b = 0; b < 8; ++b) v[b] = s_q(l1)[c][hex_node(b)];
       wht_stage(v, 4);
       wht_stage(v, 2);
       wht_stage(v, 1);
 #pragma unroll
-      for (int h = 0; h < 8; ++h) s_v(le)[h][c] = v[h];
+      for (int h = 0; h < 8; ++h) s_v(l1)[h][c] = v[h];
     }
   }
-  __syncthreads();
+  {
+    const int t1 = opaque(tid), l1 = t1 >> 3, c = t1 & 7;
+    if (LAWS != 2 || c < 2) s_c(l1)[c] = c8;
+    if (LAWS != 2 && c < 2) s_c(l1)[8 + c] = c2;
+  }
+  wave_sync();
 
-  // -- phase 2: Gauss point g of element e
+  // -- phase 2: the Gauss point of the lane's sign bits
   uint32_t fl = 0;
-  if (valid) {
-    const int gk = opaque(g);
-    // signed weights of the lane's GP: c s_gm / 8 and c^2 s_gm s_gn / 8;
-    // row i of J (i < 3) or of G_u (i = 3..5) at the GP, column k
-    auto grad_row = [&](int i, R (&out)[3]) {
-      const R c1 = (R)(0.125 * HEX_GPOS), c2 = (R)(0.125 * HEX_GPOS * HEX_GPOS);
-      const R k0 = (R)0.125;
-      const R ax = sign_if(c1, ((gk >> 2) & 1) ^ 1), ay = sign_if(c1, ((gk >> 1) & 1) ^ 1),
-              az = sign_if(c1, (gk & 1) ^ 1);
-      const R byz = sign_if(c2, ((gk >> 1) ^ gk) & 1);
-      const R bxz = sign_if(c2, ((gk >> 2) ^ gk) & 1);
-      const R bxy = sign_if(c2, ((gk >> 2) ^ (gk >> 1)) & 1);
-      const R* V7 = s_v(le)[7];
+  R Q[9], rF, detJ;
+  R qd[DAMP ? 3 : 1], zd[DAMP ? 3 : 1];   // damping terms at the point
+  {
+    const int t2 = opaque(tid), le = t2 >> 3;
+    R H[9], detF;
+    R jr[9];    // XCH: the rows of j; else j^-1
+    if constexpr (XCH) {
+      // J^-1, then row by row G_u, H = F - I = G_u J^-1 and the current
+      // Jacobian j = J + G_u = F J (J, G_u and j without HEX_SC and the column
+      // signs).  FP64: the rows of j go to LDS until the force needs their
+      // cofactors (Q = detJ tau j^-T = tau cof(j) / det F),
+      // so that neither they nor an inverse of F or j live through the law.
+      {
+        R J[9], Ji[9];  // col-major: J(i,k) = J[i + 3k]
 #pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        const int hk = 4 >> k, h1 = k == 0 ? 2 : 4, h2 = k == 2 ? 2 : 1;
-        const R w1 = k == 0 ? ay : ax, w2 = k == 2 ? ay : az, w3 = k == 0 ? byz : k == 1 ? bxz : bxy;
-        out[k] = k0 * s_v(le)[hk][i] + w1 * s_v(le)[hk | h1][i] + w2 * s_v(le)[hk | h2][i] +
-                 w3 * V7[i];
+        for (int i = 0; i < 3; ++i) {
+          R r3[3];
+          hex_grad(xr[i], r3);
+#pragma unroll
+          for (int k = 0; k < 3; ++k) J[i + 3 * k] = r3[k];
+        }
+        detJ = sma::inv3<R>(J, Ji);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          R gu[3];
+          hex_grad(xr[3 + i], gu);
+#pragma unroll
+          for (int j = 0; j < 3; ++j)
+            H[i + 3 * j] = gu[0] * Ji[3 * j] + gu[1] * Ji[1 + 3 * j] + gu[2] * Ji[2 + 3 * j];
+          if constexpr (SUR != 1) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+              if constexpr (JLDS) s_row(le)[i + 3 * k][t2 & 7] = J[i + 3 * k] + gu[k];
+              else jr[i + 3 * k] = J[i + 3 * k] + gu[k];
+            }
+          }
+        }
       }
-    };
-    // J^-1 first (J is then dead), H = F - I = G_u J^-1 (G_u row by row)
-    R Ji[9];
-    R detJ;
-    {
-      R J[9];  // col-major: J(i,k) = J[i + 3k]
+      {
+        R Fm1[9];
+#pragma unroll
+        for (int q = 0; q < 9; ++q) Fm1[q] = H[q] + ((q % 4 == 0) ? R(1) : R(0));
+        detF = sma::det3<R>(Fm1);
+      }
+    } else {
+      const int gk = t2 & 7;
+      // signed weights of the lane's GP: c s_gm / 8 and c^2 s_gm s_gn / 8;
+      // row i of J (i < 3) or of G_u (i = 3..5) at the GP, column k
+      auto grad_row = [&](int i, R (&out)[3]) {
+        const R c1 = (R)(0.125 * HEX_GPOS), c2 = (R)(0.125 * HEX_GPOS * HEX_GPOS);
+        const R k0 = (R)0.125;
+        const R ax = sign_if(c1, ((gk >> 2) & 1) ^ 1), ay = sign_if(c1, ((gk >> 1) & 1) ^ 1),
+                az = sign_if(c1, (gk & 1) ^ 1);
+        const R byz = sign_if(c2, ((gk >> 1) ^ gk) & 1);
+        const R bxz = sign_if(c2, ((gk >> 2) ^ gk) & 1);
+        const R bxy = sign_if(c2, ((gk >> 2) ^ (gk >> 1)) & 1);
+        const R* V7 = s_v(le)[7];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          const int hk = 4 >> k, h1 = k == 0 ? 2 : 4, h2 = k == 2 ? 2 : 1;
+          const R w1 = k == 0 ? ay : ax, w2 = k == 2 ? ay : az, w3 = k == 0 ? byz : k == 1 ? bxz : bxy;
+          out[k] = k0 * s_v(le)[hk][i] + w1 * s_v(le)[hk | h1][i] + w2 * s_v(le)[hk | h2][i] +
+                   w3 * V7[i];
+        }
+      };
+      // J^-1 first (J is then dead), H = F - I = G_u J^-1 (G_u row by row)
+      R Ji[9];
+      {
+        R J[9];  // col-major: J(i,k) = J[i + 3k]
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          R r3[3];
+          grad_row(i, r3);
+#pragma unroll
+          for (int k = 0; k < 3; ++k) J[i + 3 * k] = r3[k];
+        }
+        detJ = sma::inv3<R>(J, Ji);
+      }
 #pragma unroll
       for (int i = 0; i < 3; ++i) {
-        R r3[3];
-        grad_row(i, r3);
+        R gu[3];
+        grad_row(3 + i, gu);
 #pragma unroll
-        for (int k = 0; k < 3; ++k) J[i + 3 * k] = r3[k];
+        for (int j = 0; j < 3; ++j)
+          H[i + 3 * j] = gu[0] * Ji[3 * j] + gu[1] * Ji[1 + 3 * j] + gu[2] * Ji[2 + 3 * j];
       }
-      detJ = sma::inv3<R>(J, Ji);
-    }
-    R H[9];
+      // current Jacobian j = J + G_u = F J: j^-1 = J^-1 F^-1 and det j =
+      // det J det F, formed before the constitutive update
+      {
+        R Fm1[9], Fi[9];
 #pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      R gu[3];
-      grad_row(3 + i, gu);
+        for (int q = 0; q < 9; ++q) Fm1[q] = H[q] + ((q % 4 == 0) ? R(1) : R(0));
+        detF = sma::inv3<R>(Fm1, Fi);
 #pragma unroll
-      for (int j = 0; j < 3; ++j)
-        H[i + 3 * j] = gu[0] * Ji[3 * j] + gu[1] * Ji[1 + 3 * j] + gu[2] * Ji[2 + 3 * j];
-    }
-    // current Jacobian j = J + G_u = F J: j^-1 = J^-1 F^-1 and det j =
-    // det J det F, formed before the constitutive update
-    R jci[9];
-    R detF;
-    {
-      R Fm1[9], Fi[9];
+        for (int r = 0; r < 3; ++r)
 #pragma unroll
-      for (int q = 0; q < 9; ++q) Fm1[q] = H[q] + ((q % 4 == 0) ? R(1) : R(0));
-      detF = sma::inv3<R>(Fm1, Fi);
-#pragma unroll
-      for (int r = 0; r < 3; ++r)
-#pragma unroll
-        for (int c = 0; c < 3; ++c)
-          jci[r + 3 * c] = Ji[r] * Fi[3 * c] + Ji[r + 3] * Fi[1 + 3 * c] + Ji[r + 6] * Fi[2 + 3 * c];
+          for (int c = 0; c < 3; ++c)
+            jr[r + 3 * c] = Ji[r] * Fi[3 * c] + Ji[r + 3] * Fi[1 + 3 * c] + Ji[r + 6] * Fi[2 + 3 * c];
+      }
     }
 
-    if constexpr (sizeof(R) == 8) {
-      // FP64: j^-T and detJ wait in LDS through the constitutive update (the
-      // Q rows and this point's U slot are not written before it ends), so
-      // that the law runs with 20 fewer live VGPRs
-#pragma unroll
-      for (int q = 0; q < 9; ++q) s_q(le)[q][g] = jci[q];
-      s_u4(le)[g][0] = detJ;
-    }
     // det F > 0 (false for NaN); det F <= 0 stops the run (NaN is left to
     // the residual check)
     const bool detf_pos = detF > R(0);
     if constexpr (SUR != 1) {
       if (detF <= R(0)) report_detf(A.health, e, (double)detF);
     }
-    const int mat = A.mat_of_elem ? A.mat_of_elem[e] : 0;
-    const double* pr = A.props + 18 * mat;
-    const sma::Mat m = sma::make_mat_pre(pr, A.thresholds + 4 * mat, A.kg[2 * (int64_t)e],
-                                         A.kg[2 * (int64_t)e + 1]);
-    const int64_t gp = (int64_t)e * 8 + g;
-    // a neo-Hookean element has no history: its values stay as they are in
-    // both slots (equal from creation and every set), so they are neither
-    // read nor written
-    const bool neo = LAWS == 2 || (LAWS == 0 && A.law_of_elem && A.law_of_elem[e]);
-    double xS0 = 0.0, FAS0 = 0.0, FSA0 = 0.0;
-    if (!neo) {
-      xS0 = A.sdv_n[0][gp];
-      FAS0 = A.sdv_n[1][gp];
-      FSA0 = A.sdv_n[2][gp];
-    }
+    const double* pr = A.props + 18 * (int64_t)mat;   // surrogate features, mixed laws
+    sma::Mat m{};
+    if constexpr (LAWS != 2) m = sma::make_mat_const(s_c(le), s_c(le)[8], s_c(le)[9]);
 
     R tau[6];
     R Fm[9];
@@ -1071,14 +1226,17 @@ __global__ void __launch_bounds__(EPB * 8, (ElemOccupancy<R, LAWS, DAMP, STORE>:
     if (neo) {
       // neo-Hookean element: no history, no flags
       R jm1;
-      sma::neo_hookean_tau<R>(pr[0], pr[1], H, tau, jm1);
+      if constexpr (LAWS == 2) sma::neo_hookean_tau<R>(s_c(le)[0], s_c(le)[1], H, tau, jm1);
+      else sma::neo_hookean_tau<R>(pr[0], pr[1], H, tau, jm1);
       rm.xS = xS0;
       rm.F_AS = FAS0;
       rm.F_SA = FSA0;
       rm.flags = 0;
 #pragma unroll
       for (int q = 0; q < 9; ++q) Fm[q] = H[q] + ((q % 4 == 0) ? R(1) : R(0));
-      if constexpr (SUR == 1) A.sur_status[gp] = 0;
+      if constexpr (SUR == 1) {
+        if (valid) *at(A.sur_status, lb) = 0;
+      }
     } else if constexpr (sizeof(R) == 8) {
       // the Hencky tensor by series (theta, e' and e_n, no eigenvectors;
       // large stretches first halve log b by symmetric square roots)
@@ -1095,15 +1253,11 @@ __global__ void __launch_bounds__(EPB * 8, (ElemOccupancy<R, LAWS, DAMP, STORE>:
       // FP32: Hencky strain tensor by series (theta and |e'| are all the
       // return map and the stress need); the spectral form serves stretches
       // beyond the series' range
-      const sma::Hencky32 hk = sma::hencky_fp32(Hf);
+      sma::Hencky32 hk = sma::hencky_fp32(Hf);
+      bool eig_ok = true;
+      if (!hk.ok) eig_ok = sma::hencky_spectral_fp32(Hf, hk);
       if constexpr (SUR == 1) {
-        double th = hk.theta, en = hk.e_n;
-        sma::Spectral<float> sp{};
-        if (!hk.ok) {
-          sp = sma::spectral_fp32(Hf);
-          th = sp.theta;
-          en = sp.e_n;
-        }
+        const double th = hk.theta, en = hk.e_n;
         bool kf_AS, kf_SA;
         double FAS, FSA;
         const bool flagged = sma::flags_only(m, th, en, xS0, FAS0, FSA0, kf_AS, kf_SA, FAS, FSA);
@@ -1111,12 +1265,12 @@ __global__ void __launch_bounds__(EPB * 8, (ElemOccupancy<R, LAWS, DAMP, STORE>:
         // (|f| <= 8) go to the list
         float f[mlp::NIN];
         bool want = false;
-        if (flagged && kf_AS != kf_SA) {
-          // the features' principal deviatoric strains: in closed form from
-          // the series' e' (the spectral path has them already)
-          if (hk.ok) sma::principal_dev_fp32(hk.ed, sp.e[0], sp.e[1], sp.e[2]);
+        if (valid && flagged && kf_AS != kf_SA) {
+          // the features' principal deviatoric strains, in closed form
+          float e1, e2, e3;
+          sma::principal_dev_fp32(hk.ed, e1, e2, e3);
           const double E = A.E_of_elem ? A.E_of_elem[e] : pr[0];
-          mlp::make_features(pr, E, A.T_feat, sp.e[0], sp.e[1], sp.e[2], th, xS0, FAS0, FSA0, FAS, f);
+          mlp::make_features(pr, E, A.T_feat, e1, e2, e3, th, xS0, FAS0, FSA0, FAS, f);
           want = true;
 #pragma unroll
           for (int k = 0; k < mlp::NIN; ++k) want = want && fabsf(f[k]) <= 8.0f;
@@ -1139,63 +1293,127 @@ __global__ void __launch_bounds__(EPB * 8, (ElemOccupancy<R, LAWS, DAMP, STORE>:
 #pragma unroll
           for (int k = 0; k < mlp::NIN / 4; ++k)
             dst[k] = make_float4(f[4 * k], f[4 * k + 1], f[4 * k + 2], f[4 * k + 3]);
-          A.sur_slot[gp] = (int32_t)slot;
+          *at(A.sur_slot, lb) = (int32_t)slot;
         }
-        A.sur_status[gp] = !flagged ? 0 : want ? 1 : 2;
-      } else if (hk.ok) {
+        if (valid) *at(A.sur_status, lb) = !flagged ? 0 : want ? 1 : 2;
+      } else {
         if constexpr (SUR == 2) {
-          rm = surrogate_or_exact(A, m, gp, hk.theta, hk.e_n, xS0, FAS0, FSA0);
+          rm = surrogate_or_exact(A, m, (int64_t)e * 8 + lb, hk.theta, hk.e_n, xS0, FAS0, FSA0);
         } else {
           rm = sma::return_map(m, hk.theta, hk.e_n, xS0, FAS0, FSA0);
         }
         sma::kirchhoff_dev(m, hk, rm.xS, tau);
-      } else {
-        sma::Spectral<float> sp = sma::spectral_fp32(Hf);
-        if constexpr (SUR == 2) {
-          rm = surrogate_or_exact(A, m, gp, sp.theta, sp.e_n, xS0, FAS0, FSA0);
-        } else {
-          rm = sma::return_map(m, sp.theta, sp.e_n, xS0, FAS0, FSA0);
-        }
-        sma::kirchhoff<float>(m, sp, rm.xS, tau);
-        if (!sp.eig_ok) rm.flags |= sma::FLAG_EIGEN_FAIL;
+        if (!eig_ok) rm.flags |= sma::FLAG_EIGEN_FAIL;
       }
 #pragma unroll
       for (int q = 0; q < 9; ++q) Fm[q] = H[q] + ((q % 4 == 0) ? R(1) : R(0));
     }
     if constexpr (SUR != 1) {
-    if (!neo) {
-      A.sdv_k[0][gp] = rm.xS;
-      A.sdv_k[1][gp] = rm.F_AS;
-      A.sdv_k[2][gp] = rm.F_SA;
+    if (!neo && valid) {
+      *at(A.sdv_k[0], lb) = rm.xS;
+      *at(A.sdv_k[1], lb) = rm.F_AS;
+      *at(A.sdv_k[2], lb) = rm.F_SA;
     }
     fl = rm.flags;
     if (!detf_pos) fl |= sma::FLAG_DETF_NONPOS;
 
-    // Q = detJ * tau * j^-T
-    const R T[9] = {tau[0], tau[1], tau[2], tau[1], tau[3], tau[4], tau[2], tau[4], tau[5]};
-    R jq[9], dJ;
-    if constexpr (sizeof(R) == 8) {
+    const int neg = (__popc(lb) & 1) ^ 1;   // the product of the lane's signs is -1
+    R jq[9];
+    if constexpr (XCH) {
+      // Q = tau cof(j) / det F, with the constants of HEX_SC; column k keeps the
+      // factor s_gk
+      {
+        rF = sma::rcp_r(detF);
+        if constexpr (JLDS) {
+          const int t3 = opaque(tid);
 #pragma unroll
-      for (int q = 0; q < 9; ++q) jq[q] = s_q(le)[q][g];
-      dJ = s_u4(le)[g][0];
+          for (int q = 0; q < 9; ++q) jr[q] = s_row(t3 >> 3)[q][t3 & 7];
+        }
+        sma::cof3<R>(jr, jq);
+        const R sF = rF * sign_if((R)(HEX_SC * HEX_SC * HEX_SC), neg);
+        const R T[6] = {tau[0] * sF, tau[1] * sF, tau[2] * sF, tau[3] * sF, tau[4] * sF, tau[5] * sF};
+        const R Tf[9] = {T[0], T[1], T[2], T[1], T[3], T[4], T[2], T[4], T[5]};
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+#pragma unroll
+          for (int k = 0; k < 3; ++k)
+            Q[3 * i + k] = Tf[i] * jq[3 * k] + Tf[i + 3] * jq[1 + 3 * k] + Tf[i + 6] * jq[2 + 3 * k];
+      }
     } else {
+      // Q = detJ tau j^-T
+      const R T[9] = {tau[0], tau[1], tau[2], tau[1], tau[3], tau[4], tau[2], tau[4], tau[5]};
+      const int t3 = opaque(tid), l3 = t3 >> 3, g = t3 & 7;
 #pragma unroll
-      for (int q = 0; q < 9; ++q) jq[q] = jci[q];
-      dJ = detJ;
+      for (int q = 0; q < 9; ++q) jq[q] = jr[q];
+      wave_sync();
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+          s_q(l3)[3 * i + k][g] =
+              detJ * (T[i] * jq[k] + T[i + 3] * jq[k + 3] + T[i + 6] * jq[k + 6]);
     }
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-      for (int k = 0; k < 3; ++k)
-        s_q(le)[3 * i + k][g] =
-            dJ * (T[i] * jq[k] + T[i + 3] * jq[k + 3] + T[i + 6] * jq[k + 6]);
 
-    if constexpr (DAMP) {
+    if constexpr (DAMP && XCH) {
+      // Rayleigh damping at the Gauss point: q = alpha rho detJ gpvel, the
+      // velocity interpolated there (sld_elmpre.f90:110-114), and z
+      const double alpha = A.damping[2 * mat], beta = A.damping[2 * mat + 1];
+      const R arho = (R)(alpha * A.rho[mat]);
+      const R dJ = detJ * sign_if((R)(HEX_SC * HEX_SC * HEX_SC), neg);   // det J
+      constexpr double cp3 = HEX_CP * HEX_CP * HEX_CP;
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        const R gv = (R)cp3 * interp<0>(interp<1>(interp<2>(xr[6 + i])));
+        qd[i] = (R)cp3 * arho * dJ * gv;
+        zd[i] = R(0);
+      }
+      if (__ballot(beta > 0.0) != 0ull) {
+        // the beta term as written (sld_elmmat.f90:174-194):
+        // z_k = beta detJ sum_j J^-1_kj w_j, w_j = sum_k L_kj S_jk with the
+        // velocity gradient L = G_v J^-1 (gprat, sld_elmpre.f90:150-157); the
+        // exchanges of hex_grad need every lane of the element
+        R Jd[9], Gv[9];   // without HEX_SC and the column signs
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          R a3[3], b3[3];
+          hex_grad(xr[i], a3);
+          hex_grad(xr[6 + i], b3);
+#pragma unroll
+          for (int k = 0; k < 3; ++k) {
+            Jd[i + 3 * k] = a3[k];
+            Gv[i + 3 * k] = b3[k];
+          }
+        }
+        R Jid[9];
+        sma::inv3<R>(Jd, Jid);
+        R L[9], Fi[9], S[9];
+        const R rj = rF * sma::rcp_r(detJ);   // 1 / det j
+#pragma unroll
+        for (int r = 0; r < 3; ++r)
+#pragma unroll
+          for (int c = 0; c < 3; ++c) {
+            L[r + 3 * c] = Gv[r] * Jid[3 * c] + Gv[r + 3] * Jid[1 + 3 * c] + Gv[r + 6] * Jid[2 + 3 * c];
+            // F^-1 = J j^-1 (j = F J), j^-1 = cof(j)^T / det j
+            Fi[r + 3 * c] = rj * (Jd[r] * jq[c] + Jd[r + 3] * jq[c + 3] + Jd[r + 6] * jq[c + 6]);
+          }
+        sma::pk2<R>(Fi, tau, S);
+        R w[3];
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+          w[j] = L[3 * j] * S[j] + L[1 + 3 * j] * S[j + 3] + L[2 + 3 * j] * S[j + 6];
+        // z_k s_gk HEX_SC: row k of Jid is that of J^-1 times HEX_SC s_gk
+        const R bd = (R)beta * dJ;
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+          zd[k] = bd * (Jid[k] * w[0] + Jid[k + 3] * w[1] + Jid[k + 6] * w[2]);
+      }
+    }
+    if constexpr (DAMP && !XCH) {
       // Rayleigh damping at Gauss point g.  J and the velocity's natural
       // derivatives are formed again from the V(h) rows (they are not kept
       // through the constitutive update); the velocity interpolated at g is
       // gpvel = v_0 + 1/8 sum_h c^|h| s_g(h) V_v(h) (sld_elmpre.f90:110-114)
-      const int gd = opaque(g);
+      const int gd = opaque(tid) & 7, g = gd;
       const R c1 = (R)(0.125 * HEX_GPOS), c2 = (R)(0.125 * HEX_GPOS * HEX_GPOS);
       const R c3 = (R)(0.125 * HEX_GPOS * HEX_GPOS * HEX_GPOS), k0 = (R)0.125;
       const R ax = sign_if(c1, ((gd >> 2) & 1) ^ 1), ay = sign_if(c1, ((gd >> 1) & 1) ^ 1),
@@ -1214,7 +1432,7 @@ __global__ void __launch_bounds__(EPB * 8, (ElemOccupancy<R, LAWS, DAMP, STORE>:
 #pragma unroll
         for (int h = 0; h < 8; ++h) gv += wv[h] * s_v(le)[h][6 + i];
         gv += (R)s_v0[le][i];
-        s_q(le)[9 + i][g] = arho * dJ * gv;
+        s_q(le)[9 + i][g] = arho * detJ * gv;
       }
       R z[3] = {R(0), R(0), R(0)};
       if (beta > 0.0) {
@@ -1252,7 +1470,7 @@ __global__ void __launch_bounds__(EPB * 8, (ElemOccupancy<R, LAWS, DAMP, STORE>:
 #pragma unroll
         for (int j = 0; j < 3; ++j)
           w[j] = L[3 * j] * S[j] + L[1 + 3 * j] * S[j + 3] + L[2 + 3 * j] * S[j + 6];
-        const R bd = (R)beta * dJ;
+        const R bd = (R)beta * detJ;
 #pragma unroll
         for (int k = 0; k < 3; ++k)
           z[k] = bd * (Jid[k] * w[0] + Jid[k + 3] * w[1] + Jid[k + 6] * w[2]);
@@ -1265,7 +1483,8 @@ __global__ void __launch_bounds__(EPB * 8, (ElemOccupancy<R, LAWS, DAMP, STORE>:
       R Fi[9], S[9];
       sma::inv3<R>(Fm, Fi);
       sma::pk2<R>(Fi, tau, S);
-      const int64_t ngp = A.nelem * 8;
+      const int64_t ngp = A.nelem * 8, gp = (int64_t)e * 8 + lb;
+      if (valid) {
 #pragma unroll
       for (int q = 0; q < 9; ++q) A.S_out[q * ngp + gp] = (double)S[q];
       // P_jk = sum_i F_ji S_ik (sld_builtin_materials.f90:355-371), column-major
@@ -1276,6 +1495,7 @@ __global__ void __launch_bounds__(EPB * 8, (ElemOccupancy<R, LAWS, DAMP, STORE>:
           A.P_out[(j + 3 * k) * ngp + gp] =
               (double)(Fm[j] * S[3 * k] + Fm[j + 3] * S[1 + 3 * k] + Fm[j + 6] * S[2 + 3 * k]);
       A.flags_out[gp] = fl;
+      }
     }
     }  // SUR != 1
   }
@@ -1285,15 +1505,17 @@ __global__ void __launch_bounds__(EPB * 8, (ElemOccupancy<R, LAWS, DAMP, STORE>:
     // the next step's candidates: elements with a transforming point now
     if (A.sur_cand_next) {
       const unsigned long long tm = __ballot(valid && (fl & 3u));
-      if (valid && g == 0) A.sur_cand_next[e] = ((tm >> (8 * (le & 7))) & 0xffull) != 0ull;
+      if (valid && lb == 0) A.sur_cand_next[e] = ((tm >> (8 * (le & 7))) & 0xffull) != 0ull;
     }
   }
-  __syncthreads();
-  // thread g: U of Q(j = g) (Q(8) is formed in phase 3 by every thread);
-  // with damping threads 0-2 also form U of z_0..2 and threads 3-5 the
+
+
+  // Walsh-Hadamard sums: lane j forms U of Q(j) (Q(8) in phase 3, by every
+  // lane); with damping lanes 0-2 also form U of z_0..2 and lanes 3-5 the
   // Walsh-Hadamard coefficients of q_0..2
-  if (valid) {
-    const int j = opaque(g);
+  if constexpr (!XCH) {
+    const int t4 = opaque(tid), le = t4 >> 3, j = t4 & 7;
+    wave_sync();
     u4_of_q(s_q(le)[j], j % 3, s_u4(le)[j]);
     if constexpr (DAMP) {
       if (j < 3) {
@@ -1306,89 +1528,105 @@ __global__ void __launch_bounds__(EPB * 8, (ElemOccupancy<R, LAWS, DAMP, STORE>:
         wht_stage(v, 2);
         wht_stage(v, 1);
 #pragma unroll
-        for (int h = 0; h < 8; ++h) s_wq[le][j - 3][h] = v[h];
+        for (int h = 0; h < 8; ++h) s_wq(le)[j - 3][h] = v[h];
       }
     }
   }
-  __syncthreads();
 
-  // -- phase 3: thread g now owns node a = g:
-  // f_ai = sum_k s_ak/8 [U0 + c s_a1 U1 + c s_a2 U2 + c^2 s_a1 s_a2 U12](3i+k)
-  if (valid) {
-    const int a = opaque(g);
-    const int sx = (0x66 >> a) & 1, sy = (0xCC >> a) & 1, sz = (0xF0 >> a) & 1;
-    const R c0 = (R)0.125, c1 = (R)(0.125 * HEX_GPOS), c2 = (R)(0.125 * HEX_GPOS * HEX_GPOS);
-    R u8[4];
-    u4_of_q(s_q(le)[8], 2, u8);
+  // -- phase 3: the lane's corner, f_a = sum_g sum_k Q_k(g) dN_a/dxi_k(g)
+  {
     R f[3];
+    R fd[DAMP ? 3 : 1];
+    if constexpr (XCH) {
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      const int sk = k == 0 ? sx : k == 1 ? sy : sz;
-      const int s1 = k == 0 ? sy : sx, s2 = k == 2 ? sy : sz;
-      // signs s_ak, s_ak s_a1, s_ak s_a2, s_ak s_a1 s_a2 as bit parities
-      const R l0 = sign_if(c0, sk ^ 1);
-      const R l1 = sign_if(c1, sk ^ s1);
-      const R l2 = sign_if(c1, sk ^ s2);
-      const R l3 = sign_if(c2, (sk ^ s1 ^ s2) ^ 1);
+      for (int i = 0; i < 3; ++i) f[i] = hex_grad_t(Q[3 * i], Q[3 * i + 1], Q[3 * i + 2]);
+      if constexpr (DAMP) {
+        // damping force of the corner: alpha sum_g N_a(g) q(g) less the beta
+        // sum sum_g sum_k dN_a/dxi_k z_k (one value for the three components)
+        const R cb = hex_grad_t(zd[0], zd[1], zd[2]);
 #pragma unroll
-      for (int i = 0; i < 3; ++i) {
-        const R* u = (3 * i + k == 8) ? u8 : s_u4(le)[3 * i + k];
-        const R term = l0 * u[0] + l1 * u[1] + l2 * u[2] + l3 * u[3];
-        f[i] = k == 0 ? term : f[i] + term;
+        for (int i = 0; i < 3; ++i) fd[i] = interp<0>(interp<1>(interp<2>(qd[i]))) - cb;
       }
-    }
-    const R f0 = f[0], f1 = f[1], f2 = f[2];
-    if constexpr (DAMP) {
-      // damping force of corner a: alpha sum_g N_a(g) q(g) =
-      // 1/8 sum_h c^|h| s_a(h) Q_q(h), less the beta sum
-      // sum_g sum_k dN_a/dxi_k z_k (one value for the three components)
-      R cb = R(0);
+    } else {
+      // f_ai = sum_k s_ak/8 [U0 + c s_a1 U1 + c s_a2 U2 + c^2 s_a1 s_a2 U12](3i+k)
+      wave_sync();
+      const int t5 = opaque(tid), le = t5 >> 3, a = t5 & 7;
+      const int sx = (0x66 >> a) & 1, sy = (0xCC >> a) & 1, sz = (0xF0 >> a) & 1;
+      const R c0 = (R)0.125, c1 = (R)(0.125 * HEX_GPOS), c2 = (R)(0.125 * HEX_GPOS * HEX_GPOS);
+      R u8[4];
+      u4_of_q(s_q(le)[8], 2, u8);
 #pragma unroll
       for (int k = 0; k < 3; ++k) {
         const int sk = k == 0 ? sx : k == 1 ? sy : sz;
         const int s1 = k == 0 ? sy : sx, s2 = k == 2 ? sy : sz;
+        // signs s_ak, s_ak s_a1, s_ak s_a2, s_ak s_a1 s_a2 as bit parities
         const R l0 = sign_if(c0, sk ^ 1);
         const R l1 = sign_if(c1, sk ^ s1);
         const R l2 = sign_if(c1, sk ^ s2);
         const R l3 = sign_if(c2, (sk ^ s1 ^ s2) ^ 1);
-        const R* u = s_u4(le)[8 + k];
-        cb += l0 * u[0] + l1 * u[1] + l2 * u[2] + l3 * u[3];
-      }
-      const R c3 = (R)(0.125 * HEX_GPOS * HEX_GPOS * HEX_GPOS);
-      const R px = sign_if(c1, sx ^ 1), py = sign_if(c1, sy ^ 1), pz = sign_if(c1, sz ^ 1);
-      const R pyz = sign_if(c2, sy ^ sz), pxz = sign_if(c2, sx ^ sz), pxy = sign_if(c2, sx ^ sy);
-      const R pxyz = sign_if(c3, (sx ^ sy ^ sz) ^ 1);
-      const R wa[8] = {c0, pz, py, pyz, px, pxz, pxy, pxyz};
-      R fd[3];
 #pragma unroll
-      for (int i = 0; i < 3; ++i) {
-        R r = R(0);
-#pragma unroll
-        for (int h = 0; h < 8; ++h) r += wa[h] * s_wq[le][i][h];
-        fd[i] = r - cb;
+        for (int i = 0; i < 3; ++i) {
+          const R* u = (3 * i + k == 8) ? u8 : s_u4(le)[3 * i + k];
+          const R term = l0 * u[0] + l1 * u[1] + l2 * u[2] + l3 * u[3];
+          f[i] = k == 0 ? term : f[i] + term;
+        }
       }
-      R* ed = (R*)A.edamp + 3 * (int64_t)A.corner_slot[(int64_t)e * 8 + a];
-      ed[0] = fd[0];
-      ed[1] = fd[1];
-      ed[2] = fd[2];
+      if constexpr (DAMP) {
+        // damping force of corner a: alpha sum_g N_a(g) q(g) =
+        // 1/8 sum_h c^|h| s_a(h) Q_q(h), less the beta sum
+        // sum_g sum_k dN_a/dxi_k z_k (one value for the three components)
+        R cb = R(0);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          const int sk = k == 0 ? sx : k == 1 ? sy : sz;
+          const int s1 = k == 0 ? sy : sx, s2 = k == 2 ? sy : sz;
+          const R l0 = sign_if(c0, sk ^ 1);
+          const R l1 = sign_if(c1, sk ^ s1);
+          const R l2 = sign_if(c1, sk ^ s2);
+          const R l3 = sign_if(c2, (sk ^ s1 ^ s2) ^ 1);
+          const R* u = s_u4(le)[8 + k];
+          cb += l0 * u[0] + l1 * u[1] + l2 * u[2] + l3 * u[3];
+        }
+        const R c3 = (R)(0.125 * HEX_GPOS * HEX_GPOS * HEX_GPOS);
+        const R px = sign_if(c1, sx ^ 1), py = sign_if(c1, sy ^ 1), pz = sign_if(c1, sz ^ 1);
+        const R pyz = sign_if(c2, sy ^ sz), pxz = sign_if(c2, sx ^ sz), pxy = sign_if(c2, sx ^ sy);
+        const R pxyz = sign_if(c3, (sx ^ sy ^ sz) ^ 1);
+        const R wa[8] = {c0, pz, py, pyz, px, pxz, pxy, pxyz};
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          R r = R(0);
+#pragma unroll
+          for (int h = 0; h < 8; ++h) r += wa[h] * s_wq(le)[i][h];
+          fd[i] = r - cb;
+        }
+      }
+    }
+    if constexpr (DAMP) {
+      R* ed = (R*)A.edamp + 3 * (int64_t)slot;
+      if (valid) {
+        ed[0] = fd[0];
+        ed[1] = fd[1];
+        ed[2] = fd[2];
+      }
     }
     if constexpr (GATHER) {
-      R* ef = (R*)A.efor + 3 * (int64_t)A.corner_slot[(int64_t)e * 8 + a];
-      ef[0] = f0;
-      ef[1] = f1;
-      ef[2] = f2;
-    } else {
+      R* ef = (R*)A.efor + 3 * (int64_t)slot;
+      if (valid) {
+        ef[0] = f[0];
+        ef[1] = f[1];
+        ef[2] = f[2];
+      }
+    } else if (valid) {
       // coloured scatter: no other element of this colour touches this node
       R* fx = (R*)A.fint[0];
       R* fy = (R*)A.fint[1];
       R* fz = (R*)A.fint[2];
-      fx[node] += f0;
-      fy[node] += f1;
-      fz[node] += f2;
+      fx[node] += f[0];
+      fy[node] += f[1];
+      fz[node] += f[2];
     }
   }
-  // the next tile's gather writes the LDS rows phase 3 has just read
-  if (t_end - t_begin > 1) __syncthreads();
+  wave_sync();   // the next tile's gather writes the LDS rows phase 3 has just read
   }  // tile loop
 }
 

@@ -67,32 +67,34 @@ __host__ __device__ __forceinline__ Mat make_mat_kg(const double* __restrict__ p
   return m;
 }
 
-// Constants of make_mat_kg that depend on props(18) alone, per material:
-// c[0..3] = Rf_AS, Rs_AS, Rf_SA, Rs_SA (the same operations).
-__host__ __device__ __forceinline__ void mat_thresholds(const double* __restrict__ p, double* c) {
+// Constants of make_mat_kg that depend on props(18) alone, per material (the
+// same operations): c[0..7] = eL, alfa, C_AS, C_SA, Rf_AS, Rs_AS, Rf_SA, Rs_SA.
+__host__ __device__ __forceinline__ void law_constants(const double* __restrict__ p, double* c) {
   const Mat m = make_mat_kg(p, 0.0, 0.0);
-  c[0] = m.Rf_AS;
-  c[1] = m.Rs_AS;
-  c[2] = m.Rf_SA;
-  c[3] = m.Rs_SA;
+  c[0] = m.eL;
+  c[1] = m.alfa;
+  c[2] = m.C_AS;
+  c[3] = m.C_SA;
+  c[4] = m.Rf_AS;
+  c[5] = m.Rs_AS;
+  c[6] = m.Rf_SA;
+  c[7] = m.Rs_SA;
 }
 
-// make_mat_kg with the thresholds c = mat_thresholds(p) given.
-__host__ __device__ __forceinline__ Mat make_mat_pre(const double* __restrict__ p,
-                                                    const double* __restrict__ c, double K,
-                                                    double G) {
+// make_mat_kg from c = law_constants(p).
+__host__ __device__ __forceinline__ Mat make_mat_const(const double* c, double K, double G) {
 #pragma clang fp contract(off)
   Mat m;
-  m.eL = p[2];
-  m.alfa = p[14];
-  m.C_AS = p[5];
-  m.C_SA = p[11];
+  m.eL = c[0];
+  m.alfa = c[1];
+  m.C_AS = c[2];
+  m.C_SA = c[3];
   m.K = K;
   m.G = G;
-  m.Rf_AS = c[0];
-  m.Rs_AS = c[1];
-  m.Rf_SA = c[2];
-  m.Rs_SA = c[3];
+  m.Rf_AS = c[4];
+  m.Rs_AS = c[5];
+  m.Rf_SA = c[6];
+  m.Rs_SA = c[7];
   m.G_1 = (2.0 * m.G + 9.0 * (m.alfa * m.alfa) * m.K) * m.eL;
   return m;
 }
@@ -110,6 +112,41 @@ __host__ __device__ __forceinline__ float fast_rcp(float x) {
 #else
   return 1.0f / x;
 #endif
+}
+
+// 1/x in FP64 for the element step: the hardware estimate refined by two
+// Newton steps, within 1 ulp (the IEEE division: 0.5) in 5 instructions
+// against its 11.  Zero and non-finite x give NaN or infinity; a state that
+// holds one stops the run in any case.
+__host__ __device__ __forceinline__ double rcp64(double x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  double y = __builtin_amdgcn_rcp(x);
+  y = fma(fma(-x, y, 1.0), y, y);
+  return fma(fma(-x, y, 1.0), y, y);
+#else
+  return 1.0 / x;
+#endif
+}
+
+// sqrt(s) and 1/sqrt(s) of s >= 0 together: the hardware estimate refined by
+// two Newton steps (1 ulp), the root corrected once more by its residual;
+// 12 instructions against ~25 for an IEEE root and a division by it.  Below
+// 1e-290 (where the refinement would lose digits) the root is the library's
+// and its reciprocal 0 for s = 0.
+__host__ __device__ __forceinline__ void sqrt_rsqrt64(double s, double& root, double& inv) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  if (s >= 1e-290) {
+    double y = __builtin_amdgcn_rsq(s);
+    y = fma(0.5 * y, fma(-s * y, y, 1.0), y);
+    y = fma(0.5 * y, fma(-s * y, y, 1.0), y);
+    const double r = s * y;
+    root = fma(fma(-r, r, s), 0.5 * y, r);
+    inv = y;
+    return;
+  }
+#endif
+  root = sqrt(s);
+  inv = root > 0.0 ? 1.0 / root : 0.0;
 }
 
 // J^(-2/3) in FP64 (the neo-Hookean law's volumetric factor).  On the
@@ -485,30 +522,143 @@ __host__ __device__ __forceinline__ Hencky32 hencky_fp32(const float (&H)[9]) {
   return h;
 }
 
+// ---------------------------------------------------------------------------
+// The Hencky strain E = 1/2 log b = artanh(Z) = sum_k Z^(2k+1)/(2k+1),
+// Z = (b - I)(b + I)^-1, as a polynomial in Z.  By Cayley-Hamilton Z^3 = J1 Z^2
+// - J2 Z + J3 I (J1..J3 the invariants of Z), so a polynomial is three scalars
+// (on I, Z, Z^2), and a Horner step of the series, r <- Z^2 r + 1/(2k+1), is 6
+// scalar operations; a product of symmetric tensors and its sum into E, which
+// a term took before, is 30.  The identity divides by nothing, so equal or
+// nearly equal principal values need no care.  (FP64 on C1: the same count of
+// VALU instructions fell by 8% in all; measured errors of theta and e' against
+// extended precision: rms 5.5e-17 |E|, 6.5e-17 term by term.)  FP64 only: the
+// FP32 mode keeps the arithmetic its runs had, since a run amplifies a change of
+// rounding in FP32 to 2e-4 of the velocities in 200 steps.
+// ---------------------------------------------------------------------------
+
+// 1/x of the element step's precision (1 ulp)
+template <typename R>
+__host__ __device__ __forceinline__ R rcp_r(R x) {
+  if constexpr (sizeof(R) == 4) return fast_rcp(x);
+  else return rcp64(x);
+}
+
+// Z = (b - I)(b + I)^-1 from c = b - I.  With A = adj(c) and the invariants
+// I1..I3 of c, c adj(2I + c) = 4c - 2A + (2 I2 + I3) I (Cayley-Hamilton; the
+// terms of order 1 cancel in the identity, not in the arithmetic) and
+// det(2I + c) = 8 + 4 I1 + 2 I2 + I3 >= 1: 36 operations and a reciprocal,
+// without the product of c with an inverse.
+template <typename R>
+__host__ __device__ __forceinline__ void cayley(const R (&c)[6], R (&z)[6]) {
+  const R a0 = c[3] * c[5] - c[4] * c[4], a1 = c[2] * c[4] - c[1] * c[5],
+          a2 = c[1] * c[4] - c[2] * c[3], a3 = c[0] * c[5] - c[2] * c[2],
+          a4 = c[1] * c[2] - c[0] * c[4], a5 = c[0] * c[3] - c[1] * c[1];
+  const R i2 = a0 + a3 + a5, i3 = c[0] * a0 + c[1] * a1 + c[2] * a2;
+  const R q = R(2) * i2 + i3;
+  const R r = rcp_r<R>(R(8) + R(4) * (c[0] + c[3] + c[5]) + q);
+  z[0] = (R(4) * c[0] + (q - R(2) * a0)) * r;
+  z[1] = (R(4) * c[1] - R(2) * a1) * r;
+  z[2] = (R(4) * c[2] - R(2) * a2) * r;
+  z[3] = (R(4) * c[3] + (q - R(2) * a3)) * r;
+  z[4] = (R(4) * c[4] - R(2) * a4) * r;
+  z[5] = (R(4) * c[5] + (q - R(2) * a5)) * r;
+}
+
+// w = z^2 of a symmetric z; its trace is |z|_F^2.
+template <typename R>
+__host__ __device__ __forceinline__ void sym_square(const R (&z)[6], R (&w)[6]) {
+  w[0] = z[0] * z[0] + z[1] * z[1] + z[2] * z[2];
+  w[1] = z[0] * z[1] + z[1] * z[3] + z[2] * z[4];
+  w[2] = z[0] * z[2] + z[1] * z[4] + z[2] * z[5];
+  w[3] = z[1] * z[1] + z[3] * z[3] + z[4] * z[4];
+  w[4] = z[1] * z[2] + z[3] * z[4] + z[4] * z[5];
+  w[5] = z[2] * z[2] + z[4] * z[4] + z[5] * z[5];
+}
+
+// true when x holds on any active lane of the wave (on the host: for x)
+__host__ __device__ __forceinline__ bool any_lane(bool x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __ballot(x) != 0ull;
+#else
+  return x;
+#endif
+}
+
+// Horner evaluation of the series' polynomial r = a I + b Z + c Z^2.
+template <typename R>
+struct SeriesPoly {
+  R j1, j2, j3, a, b, c;
+  __host__ __device__ __forceinline__ SeriesPoly(const R (&z)[6], R zf2) {
+    j1 = z[0] + z[3] + z[5];
+    j2 = R(0.5) * (j1 * j1 - zf2);
+    j3 = z[0] * (z[3] * z[5] - z[4] * z[4]) + z[1] * (z[2] * z[4] - z[1] * z[5]) +
+         z[2] * (z[1] * z[4] - z[2] * z[3]);
+  }
+  // the two highest terms: Z^2 (w0 I) + w1 I
+  __host__ __device__ __forceinline__ void start(R w1, R w0) {
+    a = w1;
+    b = R(0);
+    c = w0;
+  }
+  // r <- Z^2 r + w I, by Z (a, b, c) = (c J3, a - c J2, b + c J1) twice
+  __host__ __device__ __forceinline__ void step(R w) {
+    const R ya = c * j3, yb = a - c * j2, yc = b + c * j1;
+    a = yc * j3 + w;
+    b = ya - yc * j2;
+    c = yb + yc * j1;
+  }
+  // E = scale Z r = e0 I + e1 Z + e2 Z^2: theta = tr E, e' = dev E, |e'|^2
+  __host__ __device__ __forceinline__ void strain(const R (&z)[6], const R (&w)[6], R zf2, R scale,
+                                                  double& theta, R (&ed)[6], R& en2) const {
+    const R e0 = scale * (c * j3), e1 = scale * (a - c * j2), e2 = scale * (b + c * j1);
+    const R t = e1 * j1 + e2 * zf2, t3 = t * R(1.0 / 3.0);
+    theta = (double)(R(3) * e0 + t);
+    ed[0] = e1 * z[0] + (e2 * w[0] - t3);
+    ed[1] = e1 * z[1] + e2 * w[1];
+    ed[2] = e1 * z[2] + e2 * w[2];
+    ed[3] = e1 * z[3] + (e2 * w[3] - t3);
+    ed[4] = e1 * z[4] + e2 * w[4];
+    ed[5] = e1 * z[5] + (e2 * w[5] - t3);
+    en2 = ed[0] * ed[0] + ed[3] * ed[3] + ed[5] * ed[5] +
+          R(2) * (ed[1] * ed[1] + ed[2] * ed[2] + ed[4] * ed[4]);
+  }
+};
+
+// The same strain by the spectral form, for stretches beyond the series'
+// range: e' = sum_k e_k n_k n_k^T.  Returns false where the eigen-solver gave
+// up.
+__host__ __device__ __forceinline__ bool hencky_spectral_fp32(const float (&H)[9], Hencky32& h) {
+  const Spectral<float> sp = spectral_fp32(H);
+  const float* n = sp.n;
+  auto sum = [&](int i, int j) {
+    return sp.e[0] * n[i] * n[j] + sp.e[1] * n[3 + i] * n[3 + j] + sp.e[2] * n[6 + i] * n[6 + j];
+  };
+  h.ed[0] = sum(0, 0);
+  h.ed[1] = sum(0, 1);
+  h.ed[2] = sum(0, 2);
+  h.ed[3] = sum(1, 1);
+  h.ed[4] = sum(1, 2);
+  h.ed[5] = sum(2, 2);
+  h.theta = sp.theta;
+  h.e_n = sp.e_n;
+  return sp.eig_ok;
+}
+
 // FP64 Hencky strain by the same series, for the plain FP64 element step:
 // E = 1/2 log b = sum_k Z^(2k+1)/(2k+1), Z = (b - I)(b + I)^-1, b - I formed
 // from H = F - I.  theta = tr E and e' = dev E are what the loading functions
 // and the stress consume (theta = log J, |e'| = e_n of compute_kirchoff_stress
 // :313-322), so no eigenvectors, square roots of eigenvalues, logarithms or
 // powers are needed; the terms run until the remainder is below 2^-54 of
-// |Z| (per lane).  Stretches with |Z|_F > 0.6 (principal stretches beyond
-// about 1/2..2) first halve the logarithm by symmetric square roots,
-// log b = 2^k log b^(1/2^k), until |Z|_F <= 0.6.
+// |Z|.  Stretches with |Z|_F > 0.6 (principal stretches beyond about 1/2..2)
+// first halve the logarithm by symmetric square roots, log b = 2^k
+// log b^(1/2^k), until |Z|_F <= 0.6.
 struct Hencky64 {
   double theta, e_n;
+  double inv_en;       // 1 / e_n (0 where e_n is 0)
   double ed[6];        // e' (00, 01, 02, 11, 12, 22)
   bool ok;             // false: no finite strain (a non-finite or non-positive b)
 };
-
-__host__ __device__ __forceinline__ void sym_mul_commuting64(const double (&a)[6],
-                                                            const double (&b)[6], double (&c)[6]) {
-  c[0] = a[0] * b[0] + a[1] * b[1] + a[2] * b[2];
-  c[1] = a[0] * b[1] + a[1] * b[3] + a[2] * b[4];
-  c[2] = a[0] * b[2] + a[1] * b[4] + a[2] * b[5];
-  c[3] = a[1] * b[1] + a[3] * b[3] + a[4] * b[4];
-  c[4] = a[1] * b[2] + a[3] * b[4] + a[4] * b[5];
-  c[5] = a[2] * b[2] + a[4] * b[4] + a[5] * b[5];
-}
 
 // Inverse of a symmetric 3x3 matrix (00, 01, 02, 11, 12, 22) by its adjugate.
 __host__ __device__ __forceinline__ void sym_inv64(const double (&m)[6], double (&r)[6]) {
@@ -521,15 +671,6 @@ __host__ __device__ __forceinline__ void sym_inv64(const double (&m)[6], double 
   const double d = 1.0 / (m[0] * r[0] + m[1] * r[1] + m[2] * r[2]);
 #pragma unroll
   for (int q = 0; q < 6; ++q) r[q] *= d;
-}
-
-// Z = (b - I)(b + I)^-1 from c = b - I; returns |Z|_F^2.
-__host__ __device__ __forceinline__ double cayley64(const double (&c)[6], double (&z)[6]) {
-  const double m[6] = {2.0 + c[0], c[1], c[2], 2.0 + c[3], c[4], 2.0 + c[5]};
-  double a[6];
-  sym_inv64(m, a);
-  sym_mul_commuting64(c, a, z);
-  return z[0] * z[0] + z[3] * z[3] + z[5] * z[5] + 2.0 * (z[1] * z[1] + z[2] * z[2] + z[4] * z[4]);
 }
 
 // Square root of a symmetric positive definite 3x3 matrix by the
@@ -556,14 +697,42 @@ __host__ __device__ __forceinline__ void sym_sqrt64(double (&y)[6]) {
   }
 }
 
-// 1/(2k+1), k = 0..40, the series' coefficients (rounded once, here, instead
-// of a division per term on the device)
-constexpr double kInvOdd64[41] = {
-    1.0 / 1,  1.0 / 3,  1.0 / 5,  1.0 / 7,  1.0 / 9,  1.0 / 11, 1.0 / 13, 1.0 / 15, 1.0 / 17,
-    1.0 / 19, 1.0 / 21, 1.0 / 23, 1.0 / 25, 1.0 / 27, 1.0 / 29, 1.0 / 31, 1.0 / 33, 1.0 / 35,
-    1.0 / 37, 1.0 / 39, 1.0 / 41, 1.0 / 43, 1.0 / 45, 1.0 / 47, 1.0 / 49, 1.0 / 51, 1.0 / 53,
-    1.0 / 55, 1.0 / 57, 1.0 / 59, 1.0 / 61, 1.0 / 63, 1.0 / 65, 1.0 / 67, 1.0 / 69, 1.0 / 71,
-    1.0 / 73, 1.0 / 75, 1.0 / 77, 1.0 / 79, 1.0 / 81};
+// Number n of series terms after Z: the remainder |Z|^(2n+3) / ((2n+3)
+// (1 - |Z|^2)) stays below 2^-54 |Z| (|Z| <= |Z|_F, zf2 = |Z|_F^2): strains
+// of 1% take 4 terms, of 5% 6; beyond 2% of zf2 the steps get coarser.  A
+// lane's n depends on its own zf2 alone, so that a point's result does not
+// depend on which points share its wave; the wave runs the Horner steps of its
+// largest n, and a lane whose series is shorter joins with its first term
+// (its coefficients before are zero, and so is its r).
+struct HenckyTerms {
+  int n;           // the wave's largest n
+  double w1, w0;   // the lane's coefficients of terms n - 1 and n
+};
+constexpr double kTerms3 = 1.4949e-04, kTerms4 = 9.0589e-04, kTerms5 = 2.9934e-03,
+                 kTerms6 = 7.0039e-03, kTerms7 = 1.3216e-02, kTerms8 = 2.1619e-02,
+                 kTerms10 = 4.4078e-02, kTerms15 = 1.1898e-01, kTerms22 = 2.2961e-01;
+__host__ __device__ __forceinline__ HenckyTerms hencky64_terms(double zf2) {
+  const bool m3 = zf2 > kTerms3;
+  if (!any_lane(m3)) return {3, 1.0 / 5, 1.0 / 7};
+  const bool m4 = zf2 > kTerms4;
+  if (!any_lane(m4)) return {4, 1.0 / 7, m3 ? 1.0 / 9 : 0.0};
+  const bool m5 = zf2 > kTerms5;
+  if (!any_lane(m5)) return {5, m3 ? 1.0 / 9 : 0.0, m4 ? 1.0 / 11 : 0.0};
+  const bool m6 = zf2 > kTerms6;
+  if (!any_lane(m6)) return {6, m4 ? 1.0 / 11 : 0.0, m5 ? 1.0 / 13 : 0.0};
+  const bool m7 = zf2 > kTerms7;
+  if (!any_lane(m7)) return {7, m5 ? 1.0 / 13 : 0.0, m6 ? 1.0 / 15 : 0.0};
+  if (!any_lane(zf2 > kTerms8)) return {8, m6 ? 1.0 / 15 : 0.0, m7 ? 1.0 / 17 : 0.0};
+  if (!any_lane(zf2 > kTerms10)) return {10, zf2 > kTerms8 ? 1.0 / 19 : 0.0, zf2 > kTerms8 ? 1.0 / 21 : 0.0};
+  if (!any_lane(zf2 > kTerms15)) return {15, zf2 > kTerms10 ? 1.0 / 29 : 0.0, zf2 > kTerms10 ? 1.0 / 31 : 0.0};
+  if (!any_lane(zf2 > kTerms22)) return {22, zf2 > kTerms15 ? 1.0 / 43 : 0.0, zf2 > kTerms15 ? 1.0 / 45 : 0.0};
+  return {32, zf2 > kTerms22 ? 1.0 / 63 : 0.0, zf2 > kTerms22 ? 1.0 / 65 : 0.0};   // zf2 <= 0.36
+}
+// 1/(2k+1), k = 7..30: the coefficients of the long series
+constexpr double kInvOdd64[24] = {
+    1.0 / 15, 1.0 / 17, 1.0 / 19, 1.0 / 21, 1.0 / 23, 1.0 / 25, 1.0 / 27, 1.0 / 29,
+    1.0 / 31, 1.0 / 33, 1.0 / 35, 1.0 / 37, 1.0 / 39, 1.0 / 41, 1.0 / 43, 1.0 / 45,
+    1.0 / 47, 1.0 / 49, 1.0 / 51, 1.0 / 53, 1.0 / 55, 1.0 / 57, 1.0 / 59, 1.0 / 61};
 
 __host__ __device__ __forceinline__ Hencky64 hencky_fp64(const double (&H)[9]) {
   Hencky64 h;
@@ -574,8 +743,10 @@ __host__ __device__ __forceinline__ Hencky64 hencky_fp64(const double (&H)[9]) {
   c[1] = H[3] + H[1] + (H[0] * H[1] + H[3] * H[4] + H[6] * H[7]);
   c[2] = H[6] + H[2] + (H[0] * H[2] + H[3] * H[5] + H[6] * H[8]);
   c[4] = H[7] + H[5] + (H[1] * H[2] + H[4] * H[5] + H[7] * H[8]);
-  double z[6];
-  double zf2 = cayley64(c, z);
+  double z[6], w[6];
+  cayley<double>(c, z);
+  sym_square<double>(z, w);
+  double zf2 = w[0] + w[3] + w[5];
   // large stretches: b <- b^(1/2) until |Z|_F <= 0.6 (each halves log b)
   int halvings = 0;
   if (zf2 > 0.36) {
@@ -584,50 +755,31 @@ __host__ __device__ __forceinline__ Hencky64 hencky_fp64(const double (&H)[9]) {
       sym_sqrt64(b);
       ++halvings;
       const double cb[6] = {b[0] - 1.0, b[1], b[2], b[3] - 1.0, b[4], b[5] - 1.0};
-      zf2 = cayley64(cb, z);
+      cayley<double>(cb, z);
+      sym_square<double>(z, w);
+      zf2 = w[0] + w[3] + w[5];
     }
   }
   h.ok = zf2 <= 0.36;
-  double e[6];
-#pragma unroll
-  for (int q = 0; q < 6; ++q) e[q] = z[q];
-  if (h.ok && zf2 > 0.0) {
-    // n terms after Z: the remainder |Z|^(2n+3)/((2n+3)(1 - |Z|^2)) stays
-    // below 2^-54 |Z| (|Z| <= |Z|_F)
-    const double lim = 5.551115123125783e-17 * (1.0 - zf2);
-    double z2[6], t[6];
-    sym_mul_commuting64(z, z, z2);
-#pragma unroll
-    for (int q = 0; q < 6; ++q) t[q] = z[q];
-    double pw = zf2;
-    for (int k = 1; k <= 40 && pw > lim * (double)(2 * k + 1); ++k) {
-      double tn[6];
-      sym_mul_commuting64(t, z2, tn);
-      const double w = kInvOdd64[k];
-#pragma unroll
-      for (int q = 0; q < 6; ++q) {
-        t[q] = tn[q];
-        e[q] += w * tn[q];
-      }
-      pw *= zf2;
-    }
+  const HenckyTerms nt = hencky64_terms(zf2);
+  const int n = nt.n;
+  SeriesPoly<double> r(z, zf2);
+  r.start(nt.w1, nt.w0);
+  if (n > 8) {
+    const int nl = zf2 > kTerms22 ? 32 : zf2 > kTerms15 ? 22 : zf2 > kTerms10 ? 15
+                 : zf2 > kTerms8 ? 10 : zf2 > kTerms7 ? 8 : zf2 > kTerms6 ? 7 : 6;
+    for (int k = n - 2; k > 6; --k) r.step(k <= nl ? kInvOdd64[k - 7] : 0.0);
   }
-  if (halvings) {
-    const double sc = (double)(1 << halvings);
-#pragma unroll
-    for (int q = 0; q < 6; ++q) e[q] *= sc;
-  }
-  const double th = e[0] + e[3] + e[5];
-  const double t3 = th * (1.0 / 3.0);
-  h.ed[0] = e[0] - t3;
-  h.ed[1] = e[1];
-  h.ed[2] = e[2];
-  h.ed[3] = e[3] - t3;
-  h.ed[4] = e[4];
-  h.ed[5] = e[5] - t3;
-  h.theta = th;
-  h.e_n = sqrt(h.ed[0] * h.ed[0] + h.ed[3] * h.ed[3] + h.ed[5] * h.ed[5] +
-               2.0 * (h.ed[1] * h.ed[1] + h.ed[2] * h.ed[2] + h.ed[4] * h.ed[4]));
+  if (n > 7) r.step(zf2 > kTerms5 ? 1.0 / 13.0 : 0.0);   // k = 6
+  if (n > 6) r.step(zf2 > kTerms4 ? 1.0 / 11.0 : 0.0);
+  if (n > 5) r.step(zf2 > kTerms3 ? 1.0 / 9.0 : 0.0);
+  if (n > 4) r.step(1.0 / 7.0);
+  if (n > 3) r.step(1.0 / 5.0);
+  r.step(1.0 / 3.0);                                     // k = 1
+  r.step(1.0);
+  double en2;
+  r.strain(z, w, zf2, (double)(1 << halvings), h.theta, h.ed, en2);
+  sqrt_rsqrt64(en2, h.e_n, h.inv_en);
   return h;
 }
 
@@ -638,7 +790,8 @@ __host__ __device__ __forceinline__ void kirchhoff_hencky64(const Mat& m, const 
                                                            double xS, double (&t)[6]) {
   const double cvol = m.K * (h.theta - 3.0 * m.alfa * m.eL * xS);
   const double twoG = 2.0 * m.G;
-  const double coef = h.e_n > 2.220446049250313080847e-16 ? twoG * (1.0 - m.eL * xS / h.e_n) : twoG;
+  const double coef =
+      h.e_n > 2.220446049250313080847e-16 ? twoG * (1.0 - m.eL * xS * h.inv_en) : twoG;
   t[0] = cvol + coef * h.ed[0];
   t[1] = coef * h.ed[1];
   t[2] = coef * h.ed[2];
@@ -745,6 +898,31 @@ __host__ __device__ __forceinline__ ReturnMap return_map(const Mat& m, double th
     double RHS_SA = (F_SA - m.Rf_SA) * dh_SA - H_SA * F_SA_dot * xS;
     double resi = RHS_AS * RHS_AS + RHS_SA * RHS_SA;   // squared first (:403)
     int iter = 0;
+    // One active branch: the other's increment and residual stay zero, the
+    // 2x2 system is its first (or second) equation, and the residual is linear
+    // in the increment, so one division solves it (the full system takes four
+    // and the inverse of a matrix).  Taken where the reference's first
+    // iteration converges as well: terms below 1e6, whose rounding (~1e-10)
+    // is far below its tolerance of 1e-8, and an idle diagonal that is not
+    // zero (the reference divides by it); else the full iteration.
+    bool done = !(resi > 1.0e-8);
+    if (!done && kf_AS != kf_SA && (kf_AS ? F_SA - m.Rf_SA : F_AS - m.Rf_AS) != 0.0) {
+      const double Rf = kf_AS ? m.Rf_AS : m.Rf_SA, F_0 = kf_AS ? F_AS_0 : F_SA_0;
+      const double F = kf_AS ? F_AS : F_SA, RHS = kf_AS ? RHS_AS : RHS_SA;
+      const double g = 0.0 - ((F - F_0) + (kf_AS ? (1.0 - xS) * m.G_1 : -(xS * m.G_1)));
+      const double dh = 0.0 - RHS / (g + (F - Rf));
+      const double x1 = xS + dh;
+      const double F1 = loading(m, kf_AS ? m.C_AS : m.C_SA, theta, e_n, x1);
+      const double t1 = (F1 - Rf) * dh, t2 = (F1 - F_0) * (kf_AS ? 1.0 - x1 : -x1);
+      if (fabs(t1 + t2) <= 1.0e-9 && fabs(t1) + fabs(t2) < 1.0e6) {
+        xS = x1;
+        F_AS = loading(m, m.C_AS, theta, e_n, xS);
+        F_SA = loading(m, m.C_SA, theta, e_n, xS);
+        iter = 1;
+        done = true;
+      }
+    }
+    if (!done)
     while (iter < 65 && resi > 1.0e-8) {
       ++iter;
       double m11 = -m.G_1 * dh_AS - (H_AS * F_AS_dot + H_AS * (1.0 - xS) * m.G_1) + (F_AS - m.Rf_AS);
@@ -856,26 +1034,37 @@ __host__ __device__ __forceinline__ void kirchhoff(const Mat& m, const Spectral<
   t[4] = c0 * n[1] * n[2] + c1 * n[4] * n[5] + c2 * n[7] * n[8];
 }
 
-// Column-major 3x3 inverse by cofactors (one reciprocal); returns det.  In
-// FP32 the reciprocal is the hardware one (1 ulp).
+// Column-major cofactor matrix: C(i,k) = d det(M) / d M(i,k), M^-1 = C^T / det.
+template <typename R>
+__host__ __device__ __forceinline__ void cof3(const R (&M)[9], R (&C)[9]) {
+  C[0] = M[4] * M[8] - M[5] * M[7];
+  C[1] = M[5] * M[6] - M[3] * M[8];
+  C[2] = M[3] * M[7] - M[4] * M[6];
+  C[3] = M[2] * M[7] - M[1] * M[8];
+  C[4] = M[0] * M[8] - M[2] * M[6];
+  C[5] = M[1] * M[6] - M[0] * M[7];
+  C[6] = M[1] * M[5] - M[2] * M[4];
+  C[7] = M[2] * M[3] - M[0] * M[5];
+  C[8] = M[0] * M[4] - M[1] * M[3];
+}
+
+template <typename R>
+__host__ __device__ __forceinline__ R det3(const R (&M)[9]) {
+  return M[0] * (M[4] * M[8] - M[5] * M[7]) + M[3] * (M[2] * M[7] - M[1] * M[8]) +
+         M[6] * (M[1] * M[5] - M[2] * M[4]);
+}
+
+// Column-major 3x3 inverse by cofactors (one reciprocal, 1 ulp); returns det.
 template <typename R>
 __host__ __device__ __forceinline__ R inv3(const R (&M)[9], R (&Mi)[9]) {
-  R c00 = M[4] * M[8] - M[5] * M[7];
-  R c01 = M[2] * M[7] - M[1] * M[8];
-  R c02 = M[1] * M[5] - M[2] * M[4];
-  R det = M[0] * c00 + M[3] * c01 + M[6] * c02;
-  R r;
-  if constexpr (sizeof(R) == 4) r = fast_rcp(det);
-  else r = R(1) / det;
-  Mi[0] = c00 * r;
-  Mi[1] = c01 * r;
-  Mi[2] = c02 * r;
-  Mi[3] = (M[5] * M[6] - M[3] * M[8]) * r;
-  Mi[4] = (M[0] * M[8] - M[2] * M[6]) * r;
-  Mi[5] = (M[2] * M[3] - M[0] * M[5]) * r;
-  Mi[6] = (M[3] * M[7] - M[4] * M[6]) * r;
-  Mi[7] = (M[1] * M[6] - M[0] * M[7]) * r;
-  Mi[8] = (M[0] * M[4] - M[1] * M[3]) * r;
+  R C[9];
+  cof3<R>(M, C);
+  const R det = M[0] * C[0] + M[3] * C[3] + M[6] * C[6];
+  const R r = rcp_r<R>(det);
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int k = 0; k < 3; ++k) Mi[i + 3 * k] = C[k + 3 * i] * r;
   return det;
 }
 

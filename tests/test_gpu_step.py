@@ -667,3 +667,20 @@ def test_fp64_step_stress_of_tiny_strains(eps):
     for k in (1, 2, 3, 5, 6, 7):
         assert np.max(np.abs(S[:, k])) < 1e-10 * sxx
     assert not np.any(fl & 3)
+
+
+@pytest.mark.parametrize("nx,ny,nz", [(1, 1, 1), (3, 1, 1), (7, 1, 1), (3, 3, 1), (11, 3, 1), (65, 1, 1)])
+@pytest.mark.parametrize("epb,assembly", [(8, "gather"), (16, "gather"), (32, "gather"), (8, "scatter")])
+def test_ragged_tiles_against_oracle(nx, ny, nz, epb, assembly):
+    """Element counts around the tile's (8 per wave, 16 and 32 per workgroup):
+    lanes past the last element repeat it and write nothing."""
+    prob = problems.cantilever_problem(nx=nx, ny=ny, nz=nz, lx=0.5 * nx, ly=0.5 * ny, lz=0.5 * nz,
+                                       nsteps=60, traction=700.0)
+    dt = prob["run"]["dt"]
+    dev, orc = _pair(prob)
+    dev.set_assembly(assembly)
+    dev.set_tile(epb)
+    dev.step(dt, nsteps=33)
+    orc.step(dt, n=33)
+    _compare(dev, orc, f"{nx}x{ny}x{nz} epb {epb} {assembly}", quiet=True)
+    dev.close()
