@@ -18,6 +18,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <type_traits>
 #include "sma_law.hpp"
 #include "surrogate_features.hpp"
 
@@ -53,7 +54,7 @@ constexpr int B_TOTAL = 4 * NH + NOUT;                           // 524
 __host__ __device__ constexpr int inf_n(int l) { return l == NLAYER - 1 ? 16 : NH; }
 static_assert(NOUT <= 16, "the output layer is one 16-feature block");
 // Inference layout of the weights (a device copy, kept by pack_params and
-// adam_step, that the inference kernel copies into LDS as it is).  Rows of
+// reduce_adam, that the inference kernel copies into LDS as it is).  Rows of
 // K + 8 BF16 (16 more bytes) per row.  An A fragment is
 // 16 rows x 16 bytes read at once; with rows of K = 128 (or 32) BF16 every
 // row starts in the same LDS bank group, and the 16 reads would queue on it.
@@ -91,176 +92,350 @@ __host__ __device__ constexpr int inf_index(int l, int n, int k) {
 __device__ __forceinline__ float silu(float z) {
   return z * __builtin_amdgcn_rcpf(1.0f + __expf(-z));
 }
-__device__ __forceinline__ float silu_grad(float z) {
-  const float s = 1.0f / (1.0f + __expf(-z));
-  return s * (1.0f + z * (1.0f - s));
+// s = sigmoid(z) to half an ulp or so (one Newton step on the hardware
+// reciprocal), silu(z) = z s and silu'(z) = s (1 + z (1 - s)).
+__device__ __forceinline__ void silu_both(float z, float& y, float& g) {
+  const float t = 1.0f + __expf(fminf(-z, 85.0f));   // finite: silu(-85) ~ 1e-35
+  float s = __builtin_amdgcn_rcpf(t);
+  y = z * s;
+  s = fmaf(fmaf(-t, s, 1.0f), s, s);
+  g = s * (1.0f + z * (1.0f - s));
 }
 
 // ----------------------------------------------------------------------------
-// Generic BF16 GEMM on MFMA: C[z][M][N] = sum_{k in chunk z} A[m][k] B[k][n]
-// A(m,k) = A[m*sam + k*sak], B(k,n) = B[k*sbk + n*sbn].  M, N multiples of 32,
-// every K chunk a multiple of 32.  One wave computes one 32x32 block.
+// Training: forward, loss, backward and weight gradients of TR_ROWS rows in one
+// workgroup, one launch per mini-batch.  What bounds it at 16384 rows (256
+// workgroups, one per CU): the chain of ~14 phases between barriers, each a
+// load or LDS read, 8 MFMA deep, an activation and an LDS write (a 1000-row
+// batch, 16 workgroups, takes 25 us; the activations are 4 us of it, the bias
+// sums 1), then writing the partial gradients (213 KB a workgroup, 54 MB, 7
+// us; reduce_adam reads them once).  Neither the 5.2 GFLOP (4 us at the rate of
+// a large BF16 product) nor the 1.8 MB of samples count.  Separate launches
+// per layer, product and activation with FP32 intermediates in memory took 930
+// us for those rows (45 launches, 0.5 GB); this takes 34, reduce_adam 14.
+// Half as many workgroups (and partials) take 1.5 times as long; loading the
+// biases, targets and output weights ahead spills and gains nothing.
+//   Products are formed as in the inference kernel (weights or their transposes
+// as the A operand), so a lane (r, q) = (lane & 15, lane >> 4) holds features
+// 4 q + i of row r of each 16x16 block: 8 waves share a layer's 128 features x
+// 64 rows as 4 x 2 blocks of 32 x 32.  silu' stays in registers (FP32) from the
+// forward to the backward pass.  LDS holds, in BF16, the layer input by rows
+// (operand of the next layer) and every layer's output and dZ by features
+// (operands of the weight gradient, whose sum runs over rows), 146 KB in all.
+//   Precision as before: BF16 weights, activations and dZ in the products, FP32
+// accumulation, FP32 Z, silu', dZ and bias gradients.
 // ----------------------------------------------------------------------------
-struct GemmArgs {
-  const __bf16* A;
-  const __bf16* B;
-  float* C;
-  int M, N, K, kchunk;
-  int64_t sam, sak, sbk, sbn;
+constexpr int TR_ROWS = 64, TR_WAVES = 8, TR_THREADS = TR_WAVES * 64;
+constexpr int TR_MAX_GRID = 256;                  // workgroups (= partial gradients)
+constexpr int GRAD_TOTAL = W_TOTAL + B_TOTAL;     // a partial gradient: canonical weights, then biases
+static_assert(GRAD_TOTAL % 4 == 0 && W_TOTAL % 4 == 0, "partials are read four at a time");
+constexpr int TR_NS = NH + 8;                     // row stride by rows (16 bytes more than 128 features)
+constexpr int TR_TS = TR_ROWS + 8;                // row stride by features
+constexpr int TR_XS = KP0 + 8;                    // row stride of the 32-wide input and output rows
+// transposed weights [k][n] of layers 1..4 (padded as the forward copy)
+__host__ __device__ constexpr int wtoff(int l) { return (l - 1) * NH * NH; }
+constexpr int WT_TOTAL = 3 * NH * NH + NH * NP4;
+
+struct TrainLds {
+  __bf16 rows[2][TR_ROWS * TR_NS];                // layer inputs, then dZ, by rows
+  __bf16 x0[TR_ROWS * TR_XS], d4[TR_ROWS * TR_XS];
+  __bf16 yt[4][NH * TR_TS];                       // Y_0..Y_3 by features
+  __bf16 t0[NH * TR_TS];                          // dZ by features
+  __bf16 x0t[NIN * TR_TS], d4t[16 * TR_TS];
+  float db[2][B_TOTAL];                           // bias gradients of the two row halves (hidden layers)
+  float db4[4][16];                               // and of the output layer's four row blocks
+  float loss[4];
 };
 
-__device__ __forceinline__ bf16x8 load8(const __bf16* p, int64_t stride) {
-  bf16x8 v;
-  if (stride == 1) {
-    v = *reinterpret_cast<const bf16x8*>(p);
-  } else {
+struct TrainArgs {
+  const __bf16* Wp;      // padded weights [n][k]
+  const __bf16* Wt;      // transposed weights of layers 1..4
+  const float* bp;
+  const float* X;        // [n][16]
+  const float* T;        // [n][12]
+  const float* w;        // loss weights
+  int64_t n;
+  int chunks;            // ceil(n / TR_ROWS); workgroup b takes chunks b, b + grid, ...
+  float* part;           // [grid][GRAD_TOTAL]
+  float* loss_part;      // [grid]
+};
+
+__device__ __forceinline__ void zero_blocks(f32x4 (&acc)[2][2]) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = p[j * stride];
+  for (int f = 0; f < 2; ++f)
+#pragma unroll
+    for (int k = 0; k < 2; ++k) acc[f][k] = f32x4{0.f, 0.f, 0.f, 0.f};
+}
+
+// A operand of a wave's 32 features of a layer (rows of K weights, 8
+// consecutive ones per lane), loaded ahead of the product that uses it
+template <int K>
+struct Weights {
+  bf16x8 a[K / 32][2];
+  __device__ __forceinline__ void load(const __bf16* A, int f0, int r, int q) {
+#pragma unroll
+    for (int c = 0; c < K / 32; ++c)
+#pragma unroll
+      for (int k = 0; k < 2; ++k)
+        a[c][k] = *reinterpret_cast<const bf16x8*>(A + (f0 + 16 * k + r) * K + 32 * c + 8 * q);
   }
+};
+
+// acc[fb][rb] = A (32 features x K) B (K x 32 rows), B rows of stride ls in LDS
+template <int K>
+__device__ __forceinline__ void block_product(f32x4 (&acc)[2][2], const Weights<K>& w, const __bf16* B, int ls,
+                                              int r0, int r, int q) {
+  zero_blocks(acc);
+#pragma unroll
+  for (int c = 0; c < K / 32; ++c) {
+    bf16x8 b[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+      b[k] = *reinterpret_cast<const bf16x8*>(B + (r0 + 16 * k + r) * ls + 32 * c + 8 * q);
+#pragma unroll
+    for (int f = 0; f < 2; ++f)
+#pragma unroll
+      for (int k = 0; k < 2; ++k)
+        acc[f][k] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.a[c][f], b[k], acc[f][k], 0, 0, 0);
+  }
+}
+
+// Workgroup barrier for LDS alone: loads of weights for the next layer and
+// stores of gradients stay in flight across it.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// sum over the 16 lanes r of a quarter wave (DPP exchanges with l ^ 1, l ^ 2,
+// l ^ 7 and l ^ 15: after each the sums of a growing group agree)
+__device__ __forceinline__ float sum16(float v) {
+  auto add = [&](auto ctrl) {
+    v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), decltype(ctrl)::value, 0xf, 0xf, true));
+  };
+  add(std::integral_constant<int, 0xB1>{});
+  add(std::integral_constant<int, 0x4E>{});
+  add(std::integral_constant<int, 0x141>{});
+  add(std::integral_constant<int, 0x140>{});
   return v;
 }
 
-__global__ void __launch_bounds__(256) gemm_bf16(GemmArgs g) {
-  const int lane = threadIdx.x & 63;
-  const int wave = (blockIdx.x * 4) + (threadIdx.x >> 6);
-  const int ntn = g.N / 32;
-  const int tm = wave / ntn, tn = wave % ntn;
-  if (tm * 32 >= g.M) return;
-  const int m0 = tm * 32, n0 = tn * 32;
-  const int z = blockIdx.z;
-  const int kbeg = z * g.kchunk, kend = min(g.K, kbeg + g.kchunk);
-  f32x4 acc[2][2];
+// 4 consecutive features of one row to the layout by rows (one 8-byte write)
+// and by features
+__device__ __forceinline__ void put4(bf16x4 h, __bf16* rows, int ls, __bf16* feat, int f, int row) {
+  if (rows) *reinterpret_cast<bf16x4*>(rows + row * ls + f) = h;
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
+  for (int i = 0; i < 4; ++i) feat[(f + i) * TR_TS + row] = h[i];
+}
+
+// weight gradient blocks: out[n][k] (+)= sum over the rows of dZ[n] Y[k], K-blocks
+// of 16 (kt by features) and one block of 16 n (dt)
+template <int NKB>
+__device__ __forceinline__ void grad_blocks(const __bf16* kt, const __bf16* dt, int k0, int n0, float* out,
+                                            int ldo, int nreal, bool first, int r, int q) {
+  const int n = n0 + r;
+  f32x4 acc[NKB];
 #pragma unroll
-    for (int b = 0; b < 2; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int r = lane & 15, kq = 8 * (lane >> 4);
-  for (int k0 = kbeg; k0 < kend; k0 += 32) {
-    bf16x8 af[2], bfr[2];
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-      af[a] = load8(g.A + (int64_t)(m0 + 16 * a + r) * g.sam + (int64_t)(k0 + kq) * g.sak, g.sak);
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-      bfr[b] = load8(g.B + (int64_t)(k0 + kq) * g.sbk + (int64_t)(n0 + 16 * b + r) * g.sbn, g.sbk);
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-      for (int b = 0; b < 2; ++b)
-        acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[a], bfr[b], acc[a][b], 0, 0, 0);
+  for (int k = 0; k < NKB; ++k) {
+    acc[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (!first && n < nreal) acc[k] = *reinterpret_cast<const f32x4*>(out + n * ldo + k0 + 16 * k + 4 * q);
   }
-  float* C = g.C + (int64_t)z * g.M * g.N;
-  const int rq = 4 * (lane >> 4);
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
+  for (int s = 0; s < TR_ROWS / 32; ++s) {
+    const bf16x8 d = *reinterpret_cast<const bf16x8*>(dt + n * TR_TS + 32 * s + 8 * q);
 #pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        C[(int64_t)(m0 + 16 * a + rq + i) * g.N + n0 + 16 * b + r] = acc[a][b][i];
-}
-
-// Sum of split-K partials in a fixed order (deterministic).
-__global__ void reduce_parts(const float* __restrict__ part, float* __restrict__ out, int64_t n, int nz) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  float s = 0.f;
-  for (int z = 0; z < nz; ++z) s += part[(int64_t)z * n + i];
-  out[i] = s;
-}
-
-// Z = C + b; hidden layers: Y = bf16(silu(Z)); output layer: Yout = Z (fp32)
-__global__ void bias_act(const float* __restrict__ C, const float* __restrict__ b, int M, int N,
-                         float* __restrict__ Z, __bf16* __restrict__ Y, int act) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (int64_t)M * N) return;
-  const int n = i % N;
-  const float z = C[i] + b[n];
-  Z[i] = z;
-  if (act) Y[i] = (__bf16)silu(z);
-}
-
-// Pack fp32 features [M][16] (rows >= n zero) into bf16 [M][32].
-__global__ void pack_input(const float* __restrict__ X, int64_t n, int M, __bf16* __restrict__ X0) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (int64_t)M * KP0) return;
-  const int64_t m = i / KP0;
-  const int k = i % KP0;
-  X0[i] = (__bf16)((m < n && k < NIN) ? X[m * NIN + k] : 0.f);
-}
-
-// Output-layer gradient of L = (1/n) sum_m sum_j w_j (y - t)^2 and the
-// per-block partial losses.
-__global__ void __launch_bounds__(256) loss_grad(const float* __restrict__ Z4, const float* __restrict__ T,
-                                                 const float* __restrict__ w, int64_t n, int M,
-                                                 float* __restrict__ dZ, __bf16* __restrict__ dZb,
-                                                 float* __restrict__ loss_part) {
-  __shared__ float red[256];
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  float l = 0.f;
-  if (i < (int64_t)M * NP4) {
-    const int64_t m = i / NP4;
-    const int j = i % NP4;
-    float g = 0.f;
-    if (m < n && j < NOUT) {
-      const float d = Z4[i] - T[m * NOUT + j];
-      l = w[j] * d * d;
-      g = 2.f * w[j] * d / (float)n;
+    for (int k = 0; k < NKB; ++k) {
+      const bf16x8 y = *reinterpret_cast<const bf16x8*>(kt + (k0 + 16 * k + r) * TR_TS + 32 * s + 8 * q);
+      acc[k] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(y, d, acc[k], 0, 0, 0);
     }
-    dZ[i] = g;
-    dZb[i] = (__bf16)g;
   }
-  red[threadIdx.x] = l;
+  if (n < nreal) {
+#pragma unroll
+    for (int k = 0; k < NKB; ++k)
+      *reinterpret_cast<f32x4*>(out + n * ldo + k0 + 16 * k + 4 * q) = acc[k];
+  }
+}
+
+__device__ __forceinline__ int opaque_index(int x) {
+  asm volatile("" : "+v"(x));
+  return x;
+}
+
+__global__ void __launch_bounds__(TR_THREADS, 2) mlp_train(TrainArgs A) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  TrainLds& S = *reinterpret_cast<TrainLds*>(smem);
+  const int tid = threadIdx.x;
+  float* part = A.part + (int64_t)blockIdx.x * GRAD_TOTAL;
+  for (int i = tid; i < 2 * B_TOTAL; i += TR_THREADS) (&S.db[0][0])[i] = 0.f;
+  if (tid < 64) (&S.db4[0][0])[tid] = 0.f;
+  for (int i = tid; i < TR_ROWS * TR_XS; i += TR_THREADS) S.d4[i] = (__bf16)0.f;
+  float loss = 0.f;
+  bool first = true;
+  for (int ch = blockIdx.x; ch < A.chunks; ch += gridDim.x, first = false) {
+    const int64_t m0 = (int64_t)ch * TR_ROWS;
+    // the thread index passes through an empty asm in every phase, so that
+    // addresses are formed where they are used and not held through the loop
+    int lane, wave, r, q, f0, rg, r0;
+    auto phase = [&]() {
+      const int t = opaque_index(tid);
+      lane = t & 63;
+      wave = __builtin_amdgcn_readfirstlane(t >> 6);
+      r = lane & 15;
+      q = lane >> 4;
+      f0 = 32 * (wave & 3);
+      rg = wave >> 2;
+      r0 = 32 * rg;
+    };
+    // inputs: 16 features a row (zero beyond the batch), 16 more of padding
+    for (int i = tid; i < TR_ROWS * KP0; i += TR_THREADS) {
+      const int row = i / KP0, k = i % KP0;
+      const __bf16 x = (__bf16)((m0 + row < A.n && k < NIN) ? A.X[(m0 + row) * NIN + k] : 0.f);
+      S.x0[row * TR_XS + k] = x;
+      if (k < NIN) S.x0t[k * TR_TS + row] = x;
+    }
+    lds_barrier();
+    f32x4 g[4][2][2];   // silu'(Z_l) of the wave's block
+    f32x4 acc[2][2];
+    // Z_l in acc -> Y_l by rows and by features, silu'(Z_l)
+    auto activate = [&](int l) {
+#pragma unroll
+      for (int f = 0; f < 2; ++f) {
+        const int feat = f0 + 16 * f + 4 * q;
+        const f32x4 b = *reinterpret_cast<const f32x4*>(A.bp + boff(l) + feat);
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          bf16x4 h;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            float y, gi;
+            silu_both(acc[f][k][i] + b[i], y, gi);
+            h[i] = (__bf16)y;
+            g[l][f][k][i] = gi;
+          }
+          put4(h, S.rows[l & 1], TR_NS, S.yt[l], feat, r0 + 16 * k + r);
+        }
+      }
+    };
+    Weights<NH> w;
+    {
+      Weights<KP0> w0;
+      phase();
+      w0.load(A.Wp + woff(0), f0, r, q);
+      w.load(A.Wp + woff(1), f0, r, q);
+      block_product<KP0>(acc, w0, S.x0, TR_XS, r0, r, q);
+      activate(0);
+      lds_barrier();
+    }
+#pragma unroll
+    for (int l = 1; l < 4; ++l) {
+      phase();
+      block_product<NH>(acc, w, S.rows[(l - 1) & 1], TR_NS, r0, r, q);
+      w.load(l < 3 ? A.Wp + woff(l + 1) : A.Wt + wtoff(3), f0, r, q);
+      activate(l);
+      lds_barrier();
+    }
+    // output layer, loss and its gradient: waves 0..3, 16 rows each
+    phase();
+    if (wave < 4) {
+      const int row = 16 * wave + r;
+      f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int c = 0; c < NH / 32; ++c) {
+        const bf16x8 a = *reinterpret_cast<const bf16x8*>(A.Wp + woff(4) + r * NH + 32 * c + 8 * q);
+        const bf16x8 b = *reinterpret_cast<const bf16x8*>(S.rows[1] + row * TR_NS + 32 * c + 8 * q);
+        o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, o, 0, 0, 0);
+      }
+      bf16x4 h;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int j = 4 * q + i;
+        float gj = 0.f;
+        if (m0 + row < A.n && j < NOUT) {
+          const float d = o[i] + A.bp[boff(4) + j] - A.T[(m0 + row) * NOUT + j];
+          loss += A.w[j] * d * d;
+          gj = 2.f * A.w[j] * d / (float)A.n;
+        }
+        h[i] = (__bf16)gj;
+        const float sj = sum16(gj);
+        if (r == 0 && j < NOUT) S.db4[wave][j] += sj;
+      }
+      put4(h, S.d4, TR_XS, S.d4t, 4 * q, row);
+    }
+    Weights<NP4> w4;
+    w4.load(A.Wt + wtoff(4), f0, r, q);
+    lds_barrier();
+    // backward: the weight gradient of layer l and dZ of layer l - 1
+    auto back = [&](int l, __bf16* rows, __bf16* feat) {
+#pragma unroll
+      for (int f = 0; f < 2; ++f) {
+        f32x4 s = {0.f, 0.f, 0.f, 0.f};
+        const int fe = f0 + 16 * f + 4 * q;
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          bf16x4 h;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const float d = acc[f][k][i] * g[l][f][k][i];
+            h[i] = (__bf16)d;
+            s[i] += d;
+          }
+          put4(h, rows, TR_NS, feat, fe, r0 + 16 * k + r);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float t = sum16(s[i]);
+          if (r == 0) S.db[rg][boff(l) + fe + i] += t;
+        }
+      }
+    };
+    phase();
+    block_product<NP4>(acc, w4, S.d4, TR_XS, r0, r, q);
+    back(3, S.rows[0], S.t0);
+    grad_blocks<1>(S.yt[3], S.d4t, 16 * wave, 0, part + woff_c(4), NH, NOUT, first, r, q);
+    lds_barrier();
+#pragma unroll
+    for (int l = 3; l >= 1; --l) {
+      // dZ_3 and dZ_1 by features lie in t0, dZ_2 and dZ_0 over Y_3 (whose last
+      // reader was the output layer's gradient)
+      const __bf16* dt = (l & 1) ? S.t0 : S.yt[3];
+      phase();
+      block_product<NH>(acc, w, S.rows[(l & 1) ^ 1], TR_NS, r0, r, q);
+      if (l > 1) w.load(A.Wt + wtoff(l - 1), f0, r, q);
+      back(l - 1, l > 1 ? S.rows[l & 1] : nullptr, (l & 1) ? S.yt[3] : S.t0);
+      phase();
+#pragma unroll
+      for (int b = 0; b < 2; ++b)   // the gradient: 32 n x 64 k a wave
+        grad_blocks<4>(S.yt[l - 1], dt, 64 * rg, f0 + 16 * b, part + woff_c(l), NH, NH, first, r, q);
+      lds_barrier();
+    }
+    phase();
+    grad_blocks<1>(S.x0t, S.yt[3], 0, 16 * wave, part + woff_c(0), NIN, NH, first, r, q);
+    lds_barrier();   // the next chunk writes x0t and Y_3
+  }
+  for (int i = tid; i < B_TOTAL; i += TR_THREADS) {
+    const int j = i - boff(4);
+    part[W_TOTAL + i] = j < 0 ? S.db[0][i] + S.db[1][i]
+                              : (S.db4[0][j] + S.db4[1][j]) + (S.db4[2][j] + S.db4[3][j]);
+  }
+  for (int d = 32; d > 0; d >>= 1) loss += __shfl_xor(loss, d);
+  if ((tid & 63) == 0 && tid < 256) S.loss[tid >> 6] = loss;
   __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) loss_part[blockIdx.x] = red[0];
+  if (tid == 0) A.loss_part[blockIdx.x] = (S.loss[0] + S.loss[1]) + (S.loss[2] + S.loss[3]);
 }
 
-// dZ = dY * silu'(Z)
-__global__ void silu_back(const float* __restrict__ dY, const float* __restrict__ Z, int64_t count,
-                          float* __restrict__ dZ, __bf16* __restrict__ dZb) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= count) return;
-  const float g = dY[i] * silu_grad(Z[i]);
-  dZ[i] = g;
-  dZb[i] = (__bf16)g;
-}
-
-// Column sums of dZ [M][N] over row chunks: part[chunk][n] (deterministic).
-__global__ void col_sums(const float* __restrict__ dZ, int M, int N, int rows_per_chunk,
-                         float* __restrict__ part) {
-  const int n = blockIdx.x * blockDim.x + threadIdx.x;
-  const int c = blockIdx.y;
-  if (n >= N) return;
-  const int r0 = c * rows_per_chunk, r1 = min(M, r0 + rows_per_chunk);
-  float s = 0.f;
-  for (int m = r0; m < r1; ++m) s += dZ[(int64_t)m * N + n];
-  part[(int64_t)c * N + n] = s;
-}
-
-// Padded gradient (layer l) -> canonical gradient layout.
-__global__ void unpad_grad(const float* __restrict__ gWp, const float* __restrict__ gbp,
-                           float* __restrict__ gW, float* __restrict__ gb, int l) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  const int K = layer_k(l), kr = layer_kreal(l), nr = layer_nreal(l);
-  if (i < nr * kr) {
-    const int n = i / kr, k = i % kr;
-    gW[woff_c(l) + i] = gWp[n * K + k];
-  }
-  if (i < nr) gb[boff(l) + i] = gbp[i];
-}
-
-// Adam on the canonical FP32 master parameters; refreshes the padded BF16
-// weights and FP32 biases the kernels read.
+// Sum of the partial gradients in a fixed order (deterministic), then Adam on
+// the canonical FP32 master parameters; refreshes the padded BF16 weights and
+// FP32 biases the kernels read.  W null: the gradient alone, to gW and gb.
+// Bound by reading the partials (54 MB at 256 workgroups): 16 threads share an
+// element's partials (a quarter of a wave reads 64 consecutive floats of one),
+// so that enough loads are in flight.
 struct AdamArgs {
+  const float* part; int parts;
   float* W; float* b;            // master, canonical
   float* mW; float* vW; float* mb; float* vb;
-  const float* gW; const float* gb;
+  float* gW; float* gb;          // gradient out (W null)
   __bf16* Wp; float* bp;         // padded device copies
   __bf16* Wi;                    // inference layout
+  __bf16* Wt;                    // transposed weights
   float lr, beta1, beta2, eps, bc1, bc2;
 };
 
@@ -271,27 +446,57 @@ __device__ __forceinline__ void adam1(float& p, float& m, float& v, float g, con
   p -= A.lr * mh / (sqrtf(vh) + A.eps);
 }
 
-__global__ void adam_step(AdamArgs A) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+constexpr int RED_ELEMS = 64;    // gradient elements per workgroup of 256
+__global__ void __launch_bounds__(256) reduce_adam(AdamArgs A) {
+  __shared__ float red[16][RED_ELEMS];
+  const int c = threadIdx.x & 15, z = threadIdx.x >> 4;
+  const int i4 = blockIdx.x * RED_ELEMS + 4 * c;
+  f32x4 s = {0.f, 0.f, 0.f, 0.f};
+  if (i4 < GRAD_TOTAL) {
+#pragma unroll 8
+    for (int p = z; p < A.parts; p += 16)
+      s += *reinterpret_cast<const f32x4*>(A.part + (int64_t)p * GRAD_TOTAL + i4);
+  }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) red[z][4 * c + k] = s[k];
+  __syncthreads();
+  if (threadIdx.x >= RED_ELEMS) return;
+  const int i = blockIdx.x * RED_ELEMS + threadIdx.x;
+  if (i >= GRAD_TOTAL) return;
+  float g = 0.f;
+#pragma unroll
+  for (int k = 0; k < 16; ++k) g += red[k][threadIdx.x];
+  if (!A.W) {
+    if (i < W_TOTAL) A.gW[i] = g;
+    else A.gb[i - W_TOTAL] = g;
+    return;
+  }
   if (i < W_TOTAL) {
-    adam1(A.W[i], A.mW[i], A.vW[i], A.gW[i], A);
+    float w = A.W[i];
+    adam1(w, A.mW[i], A.vW[i], g, A);
+    A.W[i] = w;
     int l = 0;
     while (l < 4 && i >= woff_c(l + 1)) ++l;
     const int kr = layer_kreal(l), K = layer_k(l);
     const int j = i - woff_c(l), n = j / kr, k = j % kr;
-    A.Wp[woff(l) + n * K + k] = (__bf16)A.W[i];
+    const __bf16 h = (__bf16)w;
+    A.Wp[woff(l) + n * K + k] = h;
     const int ii = inf_index(l, n, k);
-    if (ii >= 0) A.Wi[ii] = (__bf16)A.W[i];
-  }
-  if (i < B_TOTAL) {
-    adam1(A.b[i], A.mb[i], A.vb[i], A.gb[i], A);
-    A.bp[i] = A.b[i];
+    if (ii >= 0) A.Wi[ii] = h;
+    if (l > 0) A.Wt[wtoff(l) + k * layer_n(l) + n] = h;
+  } else {
+    const int k = i - W_TOTAL;
+    float w = A.b[k];
+    adam1(w, A.mb[k], A.vb[k], g, A);
+    A.b[k] = w;
+    A.bp[k] = w;
   }
 }
 
 // Canonical FP32 params -> padded device copies (pads zero).
 __global__ void pack_params(const float* __restrict__ W, const float* __restrict__ b,
-                            __bf16* __restrict__ Wp, __bf16* __restrict__ Wi, float* __restrict__ bp) {
+                            __bf16* __restrict__ Wp, __bf16* __restrict__ Wi,
+                            __bf16* __restrict__ Wt, float* __restrict__ bp) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < WPAD_TOTAL) {
     int l = 0;
@@ -302,6 +507,7 @@ __global__ void pack_params(const float* __restrict__ W, const float* __restrict
     Wp[i] = (__bf16)v;
     const int ii = inf_index(l, n, k);
     if (ii >= 0) Wi[ii] = (__bf16)v;
+    if (l > 0) Wt[wtoff(l) + k * layer_n(l) + n] = (__bf16)v;
   }
   if (i < BPAD_TOTAL) bp[i] = (i < B_TOTAL) ? b[i] : 0.f;
 }

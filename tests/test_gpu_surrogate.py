@@ -72,6 +72,29 @@ def test_gradient_matches_oracle(sur):
         o += nn * kk
 
 
+@pytest.mark.parametrize("n", [1, 16, 63, 64, 65, 129, 16384, 16385, 33001])
+def test_gradient_of_ragged_batches(sur, n):
+    """Rows around the 64 a workgroup takes, and around the 256 x 64 of one
+    pass (beyond it a workgroup adds several blocks into its partial).
+
+    Tolerance: the oracle rounds at the same points, so only roundings that FP32
+    and FP64 sums decide differently remain: a BF16 ulp (2^-8) in a small share
+    of the operands.  Weight blocks are compared by norm, at 2^-7."""
+    print(f"mlp gradient, {n} rows", flush=True)
+    rng = np.random.default_rng(n)
+    X = rng.normal(size=(n, 16)).astype(np.float32)
+    T = rng.normal(size=(n, 12)).astype(np.float32)
+    W, b = sur.get_params()
+    loss, gW, gb = sur.grad(DeviceArray.from_host(X), DeviceArray.from_host(T))
+    Lo, gWo, gbo = M.loss_and_grad(W, b, X, T, emulate=True)
+    assert abs(loss - Lo) <= 1e-3 * Lo
+    o = ob = 0
+    for (nn, kk) in M.SIZES:
+        assert _rel(gW[o:o + nn * kk], gWo[o:o + nn * kk]) < 2.0 ** -7
+        assert _rel(gb[ob:ob + nn], gbo[ob:ob + nn]) < 2.0 ** -7
+        o, ob = o + nn * kk, ob + nn
+
+
 def test_adam_step_matches_oracle():
     from alya_sma_amd.surrogate import Surrogate
     s = Surrogate(seed=9)
