@@ -10,6 +10,7 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <new>
 #include <string>
 #include <tuple>
 #include <vector>
@@ -1715,44 +1716,107 @@ int sld_dev_destroy(sld_dev* d) {
   return SMA_OK;
 }
 
-// Staging of sma160_eval, one per host thread: a device block and a pinned
-// host block, grown on demand and kept for the thread's life, so a call
-// (the reference evaluates the law once per element, 8 points) costs one
-// upload, one launch and one download instead of allocations per array.
+// Staging of sma160_eval: pinned host memory that the law kernel reads and
+// writes itself, over the host link, so that a call costs a copy into it, a
+// launch, and a copy out of it.  The law reads every input once and writes
+// every output once, in runs of 512 bytes a wave, so nothing is gained by
+// having it in device memory first: 8 points take 12 us against 32 for an
+// upload, a launch and a download (a call from Python 20 against 39).  A call
+// of more than kEvalChunk points goes through kEvalSlots slots in turn on two
+// streams: the host fills and empties slots while one kernel reads and the
+// other writes the link (40001 points: 225 us a call against 455; chunks of
+// 4096 and 16384: 288 and 295).  The material rows are read from there too (250
+// us with the 64 rows copied to the device first).
+// Memory: at most 212 bytes x kEvalChunk x kEvalSlots (5 MB) and the material
+// rows, pinned.  A call takes a stage from the pool (or makes one) and gives it
+// back; the pool keeps kEvalPool of them with blocks up to kEvalKeep, which are
+// left to the process's end (freeing after the runtime has shut down is not
+// safe).
+constexpr int64_t kEvalChunk = 6144;
+constexpr int kEvalSlots = 4, kEvalPool = 4;
+constexpr size_t kEvalKeep = (size_t)32 << 20;
 struct EvalStage {
-  void* dev = nullptr;
-  void* host = nullptr;
+  int device = -1;
+  char* host = nullptr;             // pinned; the device uses the same address
   size_t bytes = 0;
-  int device = -1;               // the device that holds `dev`
+  hipStream_t stream[2] = {nullptr, nullptr};
+  hipEvent_t done[kEvalSlots] = {nullptr, nullptr, nullptr, nullptr};
+
   int reserve(size_t want) {
-    int cur = 0;
-    HIPCHK(hipGetDevice(&cur));
-    if (cur != device) {
-      // another device is current: a block of its own (the other device's
-      // block stays with it until the process ends)
-      dev = nullptr;
-      bytes = 0;
-      device = cur;
-    }
     if (want <= bytes) return SMA_OK;
     size_t nb = bytes ? bytes : 4096;
     while (nb < want) nb *= 2;
-    if (dev) (void)hipFree(dev);
     if (host) (void)hipHostFree(host);
-    dev = host = nullptr;
+    host = nullptr;
     bytes = 0;
-    HIPCHK(hipMalloc(&dev, nb));
-    HIPCHK(hipHostMalloc(&host, nb, hipHostMallocDefault));
+    void* p = nullptr;
+    HIPCHK(hipHostMalloc(&p, nb, hipHostMallocMapped | hipHostMallocCoherent));
+    host = (char*)p;
+    HIPCHK(hipHostGetDevicePointer(&p, host, 0));
+    if (p != host) return fail(SMA_ERR_HIP, "sma160_eval: pinned memory has no common address");
     bytes = nb;
     return SMA_OK;
   }
+  int open(int dev) {
+    device = dev;
+    for (auto& q : stream) HIPCHK(hipStreamCreateWithFlags(&q, hipStreamNonBlocking));
+    for (auto& e : done) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    return SMA_OK;
+  }
+  void close() {
+    for (auto& e : done)
+      if (e) (void)hipEventDestroy(e);
+    for (auto& q : stream)
+      if (q) (void)hipStreamDestroy(q);
+    if (host) (void)hipHostFree(host);
+  }
 };
-// the blocks are left to the process's end (no destructor: freeing after
-// the runtime has shut down is not safe)
-EvalStage& eval_stage() {
-  static thread_local EvalStage* st = new EvalStage();
-  return *st;
-}
+std::mutex g_eval_mu;
+EvalStage* g_eval_pool[kEvalPool] = {};
+
+// A stage of the current device, given back (its streams idle) when the
+// call ends.
+class EvalLease {
+ public:
+  EvalStage* st = nullptr;
+  bool busy = false;                // kernels or copies may still run
+  int take() {
+    int dev = 0;
+    HIPCHK(hipGetDevice(&dev));
+    {
+      std::lock_guard<std::mutex> lock(g_eval_mu);
+      for (auto& p : g_eval_pool)
+        if (p && p->device == dev) {
+          st = p;
+          p = nullptr;
+          return SMA_OK;
+        }
+    }
+    st = new (std::nothrow) EvalStage();
+    if (!st) return fail(SMA_ERR_HIP, "sma160_eval: out of memory");
+    return st->open(dev);
+  }
+  ~EvalLease() {
+    if (!st) return;
+    if (busy)
+      for (auto& q : st->stream) (void)hipStreamSynchronize(q);
+    if (st->bytes > kEvalKeep) {
+      (void)hipHostFree(st->host);
+      st->host = nullptr;
+      st->bytes = 0;
+    }
+    {
+      std::lock_guard<std::mutex> lock(g_eval_mu);
+      for (auto& p : g_eval_pool)
+        if (!p && st->done[kEvalSlots - 1]) {
+          p = st;
+          return;
+        }
+    }
+    st->close();
+    delete st;
+  }
+};
 
 static int law_launch(int64_t n, int32_t nmat, const double* props, const int32_t* mat, const double* E,
                       const double* F, const double* sdv_old, double* sdv_new, double* S,
@@ -1791,36 +1855,83 @@ int sma160_eval(int64_t n, int32_t n_mat, const double* props, const int32_t* ma
     for (int64_t i = 0; i < n; ++i)
       if (mat_of_gp[i] < 0 || mat_of_gp[i] >= n_mat)
         return fail(SMA_ERR_ARG, "sma160_eval: material index out of range");
-  // inputs, then outputs, each section 8-byte aligned, in one block
-  const size_t b_props = (size_t)n_mat * 18 * 8, b_mat = mat_of_gp ? (size_t)((n * 4 + 7) / 8 * 8) : 0,
-               b_E = E_of_gp ? (size_t)n * 8 : 0, b_F = (size_t)n * 72, b_so = (size_t)n * 24;
-  const size_t b_sn = (size_t)n * 24, b_S = (size_t)n * 72, b_fl = flags ? (size_t)((n * 4 + 7) / 8 * 8) : 0;
-  const size_t in_bytes = b_props + b_mat + b_E + b_F + b_so, out_bytes = b_sn + b_S + b_fl;
-  EvalStage& st = eval_stage();
-  if (int rc = st.reserve(in_bytes + out_bytes)) return rc;
-  char* h = static_cast<char*>(st.host);
-  char* dv = static_cast<char*>(st.dev);
-  size_t o = 0;
-  auto put = [&](const void* src, size_t bytes, size_t span) -> size_t {
-    if (src) std::memcpy(h + o, src, bytes);
-    const size_t at = o;
-    o += span;
-    return at;
+  EvalLease lease;
+  if (int rc = lease.take()) return rc;
+  EvalStage& st = *lease.st;
+  // equal chunks of whole waves; a slot holds a chunk's sections, inputs first.
+  // A chunk's outputs are stored before a later chunk's inputs are read: fine
+  // for distinct arrays and for a call in place, one chunk for other overlaps.
+  auto meet = [&](const void* out, size_t bo, const void* in, size_t bi) {
+    const char *x = (const char*)out, *y = (const char*)in;
+    return in && x != y && x < y + bi && y < x + bo;
   };
-  const size_t o_p = put(props, b_props, b_props), o_m = put(mat_of_gp, (size_t)n * 4, b_mat);
-  const size_t o_E = put(E_of_gp, b_E, b_E), o_F = put(F, b_F, b_F), o_so = put(sdv_old, b_so, b_so);
-  const size_t o_sn = in_bytes, o_S = o_sn + b_sn, o_fl = o_S + b_S;
-  HIPCHK(hipMemcpy(dv, h, in_bytes, hipMemcpyHostToDevice));
-  auto D = [&](size_t off, size_t bytes) -> void* { return bytes ? dv + off : nullptr; };
-  if (int rc = law_launch(n, n_mat, (const double*)D(o_p, b_props), (const int32_t*)D(o_m, b_mat),
-                          (const double*)D(o_E, b_E), (const double*)D(o_F, b_F),
-                          (const double*)D(o_so, b_so), (double*)D(o_sn, b_sn), (double*)D(o_S, b_S),
-                          (uint32_t*)D(o_fl, b_fl), precision, nullptr))
-    return rc;
-  HIPCHK(hipMemcpy(h + in_bytes, dv + in_bytes, out_bytes, hipMemcpyDeviceToHost));
-  std::memcpy(sdv_new, h + o_sn, b_sn);
-  std::memcpy(S, h + o_S, b_S);
-  if (flags) std::memcpy(flags, h + o_fl, (size_t)n * 4);
+  const size_t rows = (size_t)n * 8;
+  auto meets_inputs = [&](const void* out, size_t bo) {
+    return out && (meet(out, bo, F, 9 * rows) || meet(out, bo, sdv_old, 3 * rows) ||
+                   meet(out, bo, E_of_gp, rows) || meet(out, bo, mat_of_gp, rows / 2) ||
+                   out == (const void*)E_of_gp || out == (const void*)mat_of_gp);
+  };
+  const bool whole = meets_inputs(sdv_new, 3 * rows) || meets_inputs(S, 9 * rows) ||
+                     meets_inputs(flags, rows / 2) || (const void*)sdv_new == F || (const void*)S == sdv_old;
+  int64_t nchunk = whole ? 1 : (n + kEvalChunk - 1) / kEvalChunk;
+  const int64_t per = nchunk == 1 ? n : ((n + nchunk - 1) / nchunk + 63) / 64 * 64;
+  nchunk = (n + per - 1) / per;
+  const size_t cols = (size_t)(9 + 3 + 3 + 9 + (E_of_gp ? 1 : 0));
+  const size_t slot_bytes = (size_t)per * (8 * cols + (mat_of_gp ? 4 : 0) + (flags ? 4 : 0)) + 8;
+  const size_t span = (slot_bytes + 255) / 256 * 256, b_props = (size_t)n_mat * 18 * 8;
+  const size_t head = (b_props + 255) / 256 * 256;
+  if (int rc = st.reserve(head + span * (size_t)std::min<int64_t>(nchunk, kEvalSlots))) return rc;
+  std::memcpy(st.host, props, b_props);
+  struct Slot {
+    double *F, *so, *E, *sn, *S;
+    int32_t* mat;
+    uint32_t* fl;
+  };
+  auto slot_of = [&](int64_t c) {
+    Slot q{};
+    double* d = (double*)(st.host + head + span * (size_t)(c % kEvalSlots));
+    q.F = d;
+    q.so = q.F + 9 * per;
+    q.sn = q.so + 3 * per;
+    q.S = q.sn + 3 * per;
+    d = q.S + 9 * per;
+    if (E_of_gp) q.E = d, d += per;
+    int32_t* w = (int32_t*)d;
+    if (mat_of_gp) q.mat = w, w += per;
+    if (flags) q.fl = (uint32_t*)w;
+    return q;
+  };
+  auto fill = [&](int64_t c) -> int {
+    const Slot q = slot_of(c);
+    const int64_t i0 = c * per, m = std::min(per, n - i0);
+    for (int k = 0; k < 9; ++k) std::memcpy(q.F + k * m, F + k * n + i0, (size_t)m * 8);
+    for (int k = 0; k < 3; ++k) std::memcpy(q.so + k * m, sdv_old + k * n + i0, (size_t)m * 8);
+    if (q.E) std::memcpy(q.E, E_of_gp + i0, (size_t)m * 8);
+    if (q.mat) std::memcpy(q.mat, mat_of_gp + i0, (size_t)m * 4);
+    hipStream_t s = st.stream[c & 1];
+    lease.busy = true;
+    if (int rc = law_launch(m, n_mat, (const double*)st.host, q.mat, q.E, q.F, q.so, q.sn, q.S, q.fl, precision, s))
+      return rc;
+    if (nchunk > 1) HIPCHK(hipEventRecord(st.done[c % kEvalSlots], s));
+    return SMA_OK;
+  };
+  auto drain = [&](int64_t c) -> int {
+    if (nchunk > 1) HIPCHK(hipEventSynchronize(st.done[c % kEvalSlots]));
+    else HIPCHK(hipStreamSynchronize(st.stream[0]));
+    const Slot q = slot_of(c);
+    const int64_t i0 = c * per, m = std::min(per, n - i0);
+    for (int k = 0; k < 3; ++k) std::memcpy(sdv_new + k * n + i0, q.sn + k * m, (size_t)m * 8);
+    for (int k = 0; k < 9; ++k) std::memcpy(S + k * n + i0, q.S + k * m, (size_t)m * 8);
+    if (q.fl) std::memcpy(flags + i0, q.fl, (size_t)m * 4);
+    return SMA_OK;
+  };
+  for (int64_t c = 0; c < nchunk + kEvalSlots; ++c) {
+    if (c >= kEvalSlots && c - kEvalSlots < nchunk)
+      if (int rc = drain(c - kEvalSlots)) return rc;
+    if (c < nchunk)
+      if (int rc = fill(c)) return rc;
+  }
+  lease.busy = false;
   return SMA_OK;
 }
 

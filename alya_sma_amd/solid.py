@@ -23,6 +23,11 @@ def _p(a):
     return None if a is None else a.ctypes.data_as(C.c_void_p)
 
 
+def _addr(a):
+    """Address of an array that the caller holds through the call."""
+    return None if a is None else a.__array_interface__["data"][0]
+
+
 def _c(a, dt):
     return None if a is None else np.ascontiguousarray(a, dtype=dt)
 
@@ -39,13 +44,13 @@ def eval_sld_stress_model_160(props, F, sdv_old, mat_of_gp=None, E_of_gp=None, p
     n = F.shape[1]
     if F.shape != (9, n) or sdv_old.shape != (3, n):
         raise ValueError("F must be [9, n] and sdv_old [3, n]")
-    sdv_new = np.zeros((3, n))
-    S = np.zeros((9, n))
-    flags = np.zeros(n, dtype=np.uint32)
+    sdv_new = np.empty((3, n))
+    S = np.empty((9, n))
+    flags = np.empty(n, dtype=np.uint32)
     mat = _c(mat_of_gp, np.int32)
     E = _c(E_of_gp, np.float64)
-    check(lib().sma160_eval(n, props.shape[0], _p(props), _p(mat), _p(E), _p(F), None,
-                            _p(sdv_old), _p(sdv_new), _p(S), _p(flags), int(precision)),
+    check(lib().sma160_eval(n, props.shape[0], _addr(props), _addr(mat), _addr(E), _addr(F), None,
+                            _addr(sdv_old), _addr(sdv_new), _addr(S), _addr(flags), int(precision)),
           "sma160_eval")
     return sdv_new, S, flags
 
