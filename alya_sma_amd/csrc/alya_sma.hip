@@ -56,12 +56,13 @@ constexpr int GRAPH_RUNS[] = {64, 16, 2};
 
 struct GraphKey {
   double dt, phi;
-  int scheme, mode, store, epb, xcd, persistent, assembly, tn, energy, len, damp, body;
+  int scheme, mode, store, epb, xcd, persistent, assembly, tn, energy, len, damp, body, one_f;
   bool operator<(const GraphKey& o) const {
     return std::tie(dt, phi, scheme, mode, store, epb, xcd, persistent, assembly, tn, energy, len,
-                    damp, body) <
+                    damp, body, one_f) <
            std::tie(o.dt, o.phi, o.scheme, o.mode, o.store, o.epb, o.xcd, o.persistent,
-                    o.assembly, o.tn, o.energy, o.len, o.damp, o.body);
+                    o.assembly, o.tn, o.energy, o.len, o.damp, o.body,
+                    o.one_f);
   }
 };
 
@@ -110,6 +111,16 @@ struct sld_dev {
   uint8_t* law_of_elem = nullptr;    // [nelem] 1 = neo-Hookean; null when all SMA
   int32_t nh_begin = -1;             // first stored neo-Hookean element (law-grouped), or -1
   double* sdv[2][3] = {};
+  // One loading function for both branches.  The law's F_AS and F_SA differ
+  // only by C_AS and C_SA times a temperature that is 0, so once equal they stay
+  // equal to the last bit (both are the loading function at the new xS, or both
+  // keep their old value); a run at rest starts with both 0.  While `one_f` is
+  // set the element launches read and write F_AS alone (the third history
+  // pointer is the second), 16 of a point's 48 bytes less; the array of F_SA
+  // is then current only for neo-Hookean elements, which no launch touches.
+  // Unset by a history whose two values differ, or constants that are not
+  // finite.
+  bool one_f = false, finite_c = false;
   int cur = 1;                       // index of the TIME_N history and clock slot
   double* S_out = nullptr;
   double* P_out = nullptr;
@@ -473,6 +484,10 @@ int enqueue_step(sld_dev* d, double dt, int scheme, double phi, int tn, KernelTi
       E.sdv_n[k] = d->sdv[tn][k];
       E.sdv_k[k] = d->sdv[1 - tn][k];
       E.fint[k] = N.fint[k];
+    }
+    if (d->one_f) {
+      E.sdv_n[2] = E.sdv_n[1];
+      E.sdv_k[2] = E.sdv_k[1];
     }
     E.efor = d->efor;
     E.corner_slot = d->corner_slot;
@@ -862,6 +877,10 @@ int sld_dev_create(const sld_mesh_desc* mesh, const sld_material_desc* mat,
     std::vector<double> lc((size_t)mat->nmat * 8);
     for (int k = 0; k < mat->nmat; ++k) sma::law_constants(mat->props + 18 * (size_t)k, &lc[8 * (size_t)k]);
     TRY(upload(&d->law_const, lc.data(), lc.size(), s)); track(d, d->law_const);
+    d->finite_c = true;
+    for (int k = 0; k < mat->nmat; ++k)
+      d->finite_c = d->finite_c && std::isfinite(lc[8 * (size_t)k + 2]) && std::isfinite(lc[8 * (size_t)k + 3]);
+    d->one_f = d->finite_c;
   }
   TRY(upload(&d->rho, mat->rho, (size_t)mat->nmat, s)); track(d, d->rho);
   std::vector<int32_t> me;
@@ -1200,7 +1219,7 @@ int sld_dev_energy(sld_dev* d, double* out) {
 // handle's current settings, built on first use and kept.
 static int run_graph(sld_dev* d, double dt, int32_t scheme, double phi, int len, hipGraphExec_t* out) {
   GraphKey key{dt, phi, scheme, d->mode, d->store, d->epb, d->xcd, d->persistent, d->assembly, d->cur,
-               d->energy, len, d->damp, d->body_func};
+               d->energy, len, d->damp, d->body_func, d->one_f};
   auto it = d->graphs.find(key);
   if (it == d->graphs.end()) {
     hipGraph_t g = nullptr;
@@ -1504,7 +1523,15 @@ int sld_dev_get(sld_dev* d, int32_t field, void* host, int64_t count) {
       const int k_slot = d->cur;  // after a step the slot just written holds TIME_N = ITER_K
       tmp.resize(ngp);
       for (int k = 0; k < 3; ++k) {
-        HIPCHK(hipMemcpy(tmp.data(), d->sdv[k_slot][k], ngp * sizeof(double), hipMemcpyDeviceToHost));
+        if (k == 2 && d->one_f) {
+          // F_SA of the SMA elements (stored first) is F_AS, still in tmp
+          const int64_t sma = 8 * (int64_t)(d->nh_begin >= 0 ? d->nh_begin : ne);
+          if (ngp > sma)
+            HIPCHK(hipMemcpy(tmp.data() + sma, d->sdv[k_slot][k] + sma, (ngp - sma) * sizeof(double),
+                             hipMemcpyDeviceToHost));
+        } else {
+          HIPCHK(hipMemcpy(tmp.data(), d->sdv[k_slot][k], ngp * sizeof(double), hipMemcpyDeviceToHost));
+        }
         for (int64_t i = 0; i < ne; ++i)
           for (int g = 0; g < 8; ++g) out[(8 * (int64_t)d->order[i] + g) * 3 + k] = tmp[8 * i + g];
       }
@@ -1638,6 +1665,13 @@ int sld_dev_set(sld_dev* d, int32_t field, const void* host, int64_t count) {
       if (count != 3 * ngp) return fail(SMA_ERR_ARG, "count does not match field size");
       const double* in = (const double*)host;
       tmp.resize(ngp);
+      const int64_t nsma = d->nh_begin >= 0 ? d->nh_begin : ne;
+      d->one_f = d->finite_c;
+      for (int64_t i = 0; i < nsma && d->one_f; ++i)
+        for (int g = 0; g < 8; ++g) {
+          const double* f = in + (8 * (int64_t)d->order[i] + g) * 3;
+          d->one_f = d->one_f && std::memcmp(f + 1, f + 2, sizeof(double)) == 0;
+        }
       for (int k = 0; k < 3; ++k) {
         for (int64_t i = 0; i < ne; ++i)
           for (int g = 0; g < 8; ++g) tmp[8 * i + g] = in[(8 * (int64_t)d->order[i] + g) * 3 + k];
