@@ -74,6 +74,7 @@ struct sld_dev {
   std::vector<int32_t> color_ptr;   // [ncolor+1] ranges of color_list
   std::vector<int32_t> color_list;  // stored elements sorted by colour (stable)
   std::vector<int32_t> order;       // stored position -> caller element
+  int32_t* stored_dev = nullptr;    // caller element -> stored position (null: the same), for read-back
   int32_t* color_list_dev = nullptr;
   // device arrays
   int32_t* lnods = nullptr;
@@ -582,6 +583,184 @@ int enqueue_step(sld_dev* d, double dt, int scheme, double phi, int tn, KernelTi
   TEND();
   HIPCHK(hipGetLastError());
   return 0;
+}
+
+// Staging of host arrays: pinned memory that kernels read and write themselves,
+// over the host link, so that operands and results need no copy of their own.
+// A transfer goes through kStageSlots slots in turn on two streams: the host
+// fills and empties slots while kernels read and write others.  A call takes a
+// stage from the pool (or makes one) and gives it back; the pool keeps kStagePool
+// of them with blocks up to kStageKeep, which are left to the process's end
+// (freeing after the runtime has shut down is not safe).
+constexpr int kStageSlots = 4, kStagePool = 4;
+constexpr size_t kStageKeep = (size_t)32 << 20;
+struct HostStage {
+  int device = -1;
+  char* host = nullptr;             // pinned; the device uses the same address
+  size_t bytes = 0;
+  hipStream_t stream[2] = {nullptr, nullptr};
+  hipEvent_t done[kStageSlots] = {nullptr, nullptr, nullptr, nullptr};
+
+  int reserve(size_t want) {
+    if (want <= bytes) return SMA_OK;
+    size_t nb = bytes ? bytes : 4096;
+    while (nb < want) nb *= 2;
+    if (host) (void)hipHostFree(host);
+    host = nullptr;
+    bytes = 0;
+    void* p = nullptr;
+    HIPCHK(hipHostMalloc(&p, nb, hipHostMallocMapped | hipHostMallocCoherent));
+    host = (char*)p;
+    HIPCHK(hipHostGetDevicePointer(&p, host, 0));
+    if (p != host) return fail(SMA_ERR_HIP, "host stage: pinned memory has no common address");
+    bytes = nb;
+    return SMA_OK;
+  }
+  int open(int dev) {
+    device = dev;
+    for (auto& q : stream) HIPCHK(hipStreamCreateWithFlags(&q, hipStreamNonBlocking));
+    for (auto& e : done) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    return SMA_OK;
+  }
+  void close() {
+    for (auto& e : done)
+      if (e) (void)hipEventDestroy(e);
+    for (auto& q : stream)
+      if (q) (void)hipStreamDestroy(q);
+    if (host) (void)hipHostFree(host);
+  }
+};
+std::mutex g_stage_mu;
+HostStage* g_stage_pool[kStagePool] = {};
+
+// A stage of the current device, given back (its streams idle) when the
+// call ends.
+class HostLease {
+ public:
+  HostStage* st = nullptr;
+  bool busy = false;                // kernels or copies may still run
+  int take() {
+    int dev = 0;
+    HIPCHK(hipGetDevice(&dev));
+    {
+      std::lock_guard<std::mutex> lock(g_stage_mu);
+      for (auto& p : g_stage_pool)
+        if (p && p->device == dev) {
+          st = p;
+          p = nullptr;
+          return SMA_OK;
+        }
+    }
+    st = new (std::nothrow) HostStage();
+    if (!st) return fail(SMA_ERR_HIP, "host stage: out of memory");
+    return st->open(dev);
+  }
+  ~HostLease() {
+    if (!st) return;
+    if (busy)
+      for (auto& q : st->stream) (void)hipStreamSynchronize(q);
+    if (st->bytes > kStageKeep) {
+      (void)hipHostFree(st->host);
+      st->host = nullptr;
+      st->bytes = 0;
+    }
+    {
+      std::lock_guard<std::mutex> lock(g_stage_mu);
+      for (auto& p : g_stage_pool)
+        if (!p && st->done[kStageSlots - 1]) {
+          p = st;
+          return;
+        }
+    }
+    st->close();
+    delete st;
+  }
+};
+
+// The handle's device, made current for a scope.
+struct DeviceScope {
+  int before = -1, now = -1;
+  int enter(int dev) {
+    HIPCHK(hipGetDevice(&before));
+    now = before;
+    if (dev != before) {
+      HIPCHK(hipSetDevice(dev));
+      now = dev;
+    }
+    return 0;
+  }
+  ~DeviceScope() {
+    if (now != before) (void)hipSetDevice(before);
+  }
+};
+
+// Uploads the stored position of each element when it differs (once).
+int stored_positions(sld_dev* d) {
+  if (d->stored_dev || d->nh_begin < 0) return 0;
+  std::vector<int32_t> pos((size_t)d->nelem);
+  for (int64_t i = 0; i < d->nelem; ++i) pos[d->order[i]] = (int32_t)i;
+  int32_t* p = nullptr;
+  if (int rc = upload(&p, pos.data(), pos.size(), d->stream)) return rc;
+  track(d, p);
+  d->stored_dev = p;
+  return 0;
+}
+
+// Rows of a result from the device to the caller's array: `launch` packs rows
+// row0 .. row0 + m - 1 into a slot of the stage, the host copies them out.
+// Before, each component was copied to a host vector and the components
+// interleaved by host loops: u of 695 000 nodes 2.1 ms, now 0.64; the history
+// of 5.05 million points 28 ms, now 8.2 (most of it the caller's fresh pages).
+constexpr size_t kPackSlot = (size_t)1 << 20;
+template <class Launch>
+int staged_rows(const sld_dev* d, int64_t rows, size_t row_bytes, char* out, Launch launch) {
+  if (rows == 0) return 0;
+  DeviceScope scope;
+  if (int rc = scope.enter(d->device)) return rc;
+  HostLease lease;
+  if (int rc = lease.take()) return rc;
+  HostStage& st = *lease.st;
+  const int64_t per = std::min<int64_t>(rows, (int64_t)(kPackSlot / row_bytes));
+  const int64_t nchunk = (rows + per - 1) / per;
+  const size_t span = ((size_t)per * row_bytes + 255) / 256 * 256;
+  if (int rc = st.reserve(span * (size_t)std::min<int64_t>(nchunk, kStageSlots))) return rc;
+  lease.busy = true;
+  for (int64_t c = 0; c < nchunk + kStageSlots; ++c) {
+    const int64_t e = c - kStageSlots;
+    char* slot = st.host + span * (size_t)(c % kStageSlots);
+    if (e >= 0 && e < nchunk) {
+      HIPCHK(hipEventSynchronize(st.done[e % kStageSlots]));
+      std::memcpy(out + (size_t)(e * per) * row_bytes, slot, (size_t)std::min(per, rows - e * per) * row_bytes);
+    }
+    if (c < nchunk) {
+      hipStream_t s = st.stream[c & 1];
+      launch(c * per, std::min(per, rows - c * per), (double*)slot, s);
+      HIPCHK(hipGetLastError());
+      HIPCHK(hipEventRecord(st.done[c % kStageSlots], s));
+    }
+  }
+  lease.busy = false;
+  return 0;
+}
+
+// NC components of a field (arrays of double, or of float), by rows; with
+// `stored`, rows are Gauss points of the caller's elements; the third component
+// of the first `same` stored rows is the second.
+template <int NC>
+int get_rows(const sld_dev* d, const void* const (&src)[NC], bool fp32, const int32_t* stored, int64_t rows,
+             void* out, int64_t same = 0) {
+  sld::PackArgs A{};
+  A.same = same;
+  for (int k = 0; k < NC; ++k) A.src[k] = src[k];
+  A.fp32 = fp32 ? 1 : 0;
+  A.stored = stored;
+  return staged_rows(d, rows, NC * sizeof(double), (char*)out, [&](int64_t row0, int64_t m, double* slot,
+                                                                 hipStream_t s) {
+    A.row0 = row0;
+    A.rows = (int32_t)m;
+    A.out = slot;
+    hipLaunchKernelGGL((sld::sld_pack<NC>), dim3(nblocks(m * NC, 256)), dim3(256), 0, s, A);
+  });
 }
 
 void free_graphs(sld_dev* d) {
@@ -1497,21 +1676,12 @@ int sld_dev_get(sld_dev* d, int32_t field, void* host, int64_t count) {
   switch (field) {
     case SLD_FIELD_U: case SLD_FIELD_V: case SLD_FIELD_A: case SLD_FIELD_FINT: {
       if (need(3 * np)) return SMA_ERR_ARG;
-      double* out = (double*)host;
-      tmp.resize(np);
-      for (int k = 0; k < 3; ++k) {
-        if (field == SLD_FIELD_FINT && d->mode != SLD_MODE_FP64) {
-          std::vector<float> t32(np);
-          HIPCHK(hipMemcpy(t32.data(), d->fint32[k], np * sizeof(float), hipMemcpyDeviceToHost));
-          for (int64_t p = 0; p < np; ++p) tmp[p] = t32[p];
-        } else {
-          double* src = field == SLD_FIELD_U ? d->u[k] : field == SLD_FIELD_V ? d->v[k]
-                      : field == SLD_FIELD_A ? d->a[k] : d->fint64[k];
-          HIPCHK(hipMemcpy(tmp.data(), src, np * sizeof(double), hipMemcpyDeviceToHost));
-        }
-        for (int64_t p = 0; p < np; ++p) out[3 * p + k] = tmp[p];
-      }
-      return SMA_OK;
+      const bool f32 = field == SLD_FIELD_FINT && d->mode != SLD_MODE_FP64;
+      const void* src[3];
+      for (int k = 0; k < 3; ++k)
+        src[k] = field == SLD_FIELD_U ? (void*)d->u[k] : field == SLD_FIELD_V ? (void*)d->v[k]
+               : field == SLD_FIELD_A ? (void*)d->a[k] : f32 ? (void*)d->fint32[k] : (void*)d->fint64[k];
+      return get_rows<3>(d, src, f32, nullptr, np, host);
     }
     case SLD_FIELD_MASS:
       if (need(np)) return SMA_ERR_ARG;
@@ -1519,23 +1689,12 @@ int sld_dev_get(sld_dev* d, int32_t field, void* host, int64_t count) {
       return SMA_OK;
     case SLD_FIELD_SDV: {
       if (need(3 * ngp)) return SMA_ERR_ARG;
-      double* out = (double*)host;
       const int k_slot = d->cur;  // after a step the slot just written holds TIME_N = ITER_K
-      tmp.resize(ngp);
-      for (int k = 0; k < 3; ++k) {
-        if (k == 2 && d->one_f) {
-          // F_SA of the SMA elements (stored first) is F_AS, still in tmp
-          const int64_t sma = 8 * (int64_t)(d->nh_begin >= 0 ? d->nh_begin : ne);
-          if (ngp > sma)
-            HIPCHK(hipMemcpy(tmp.data() + sma, d->sdv[k_slot][k] + sma, (ngp - sma) * sizeof(double),
-                             hipMemcpyDeviceToHost));
-        } else {
-          HIPCHK(hipMemcpy(tmp.data(), d->sdv[k_slot][k], ngp * sizeof(double), hipMemcpyDeviceToHost));
-        }
-        for (int64_t i = 0; i < ne; ++i)
-          for (int g = 0; g < 8; ++g) out[(8 * (int64_t)d->order[i] + g) * 3 + k] = tmp[8 * i + g];
-      }
-      return SMA_OK;
+      const void* src[3] = {d->sdv[k_slot][0], d->sdv[k_slot][1], d->sdv[k_slot][2]};
+      // F_SA of the SMA elements (stored first) is F_AS
+      const int64_t same = !d->one_f ? 0 : 8 * (int64_t)(d->nh_begin >= 0 ? d->nh_begin : ne);
+      if (int rc = stored_positions(d)) return rc;
+      return get_rows<3>(d, src, false, d->stored_dev, ngp, host, same);
     }
     case SLD_FIELD_REACTIONS: {
       if (need(3 * np)) return SMA_ERR_ARG;
@@ -1580,15 +1739,11 @@ int sld_dev_get(sld_dev* d, int32_t field, void* host, int64_t count) {
     case SLD_FIELD_STRESS: case SLD_FIELD_PK1: {
       if (!d->S_out) return fail(SMA_ERR_STATE, "stress not stored (sld_dev_set_store)");
       if (need(9 * ngp)) return SMA_ERR_ARG;
-      double* out = (double*)host;
-      tmp.resize(9 * ngp);
-      HIPCHK(hipMemcpy(tmp.data(), field == SLD_FIELD_PK1 ? d->P_out : d->S_out,
-                       9 * ngp * sizeof(double), hipMemcpyDeviceToHost));
-      for (int k = 0; k < 9; ++k)
-        for (int64_t i = 0; i < ne; ++i)
-          for (int g = 0; g < 8; ++g)
-            out[(8 * (int64_t)d->order[i] + g) * 9 + k] = tmp[k * ngp + 8 * i + g];
-      return SMA_OK;
+      const double* f = field == SLD_FIELD_PK1 ? d->P_out : d->S_out;
+      const void* src[9];
+      for (int k = 0; k < 9; ++k) src[k] = f + k * ngp;
+      if (int rc = stored_positions(d)) return rc;
+      return get_rows<9>(d, src, false, d->stored_dev, ngp, host);
     }
     case SLD_FIELD_FLAGS: {
       if (!d->flags_out) return fail(SMA_ERR_STATE, "flags not stored (sld_dev_set_store)");
@@ -1750,107 +1905,15 @@ int sld_dev_destroy(sld_dev* d) {
   return SMA_OK;
 }
 
-// Staging of sma160_eval: pinned host memory that the law kernel reads and
-// writes itself, over the host link, so that a call costs a copy into it, a
-// launch, and a copy out of it.  The law reads every input once and writes
-// every output once, in runs of 512 bytes a wave, so nothing is gained by
-// having it in device memory first: 8 points take 12 us against 32 for an
-// upload, a launch and a download (a call from Python 20 against 39).  A call
-// of more than kEvalChunk points goes through kEvalSlots slots in turn on two
-// streams: the host fills and empties slots while one kernel reads and the
-// other writes the link (40001 points: 225 us a call against 455; chunks of
-// 4096 and 16384: 288 and 295).  The material rows are read from there too (250
-// us with the 64 rows copied to the device first).
-// Memory: at most 212 bytes x kEvalChunk x kEvalSlots (5 MB) and the material
-// rows, pinned.  A call takes a stage from the pool (or makes one) and gives it
-// back; the pool keeps kEvalPool of them with blocks up to kEvalKeep, which are
-// left to the process's end (freeing after the runtime has shut down is not
-// safe).
+// sma160_eval's points go through a stage: the law reads every input once and
+// writes every output once, in runs of 512 bytes a wave, so nothing is gained by
+// having them in device memory first.  8 points take 12 us against 32 for an
+// upload, a launch and a download (a call from Python 20 against 39); 40001
+// points, in chunks, 225 us a call against 455 (chunks of 4096 and 16384: 288
+// and 295).  The material rows are read from there too (250 us with the 64 rows
+// copied to the device first).
+// Memory: at most 212 bytes x kEvalChunk x kStageSlots (5 MB) and the material rows.
 constexpr int64_t kEvalChunk = 6144;
-constexpr int kEvalSlots = 4, kEvalPool = 4;
-constexpr size_t kEvalKeep = (size_t)32 << 20;
-struct EvalStage {
-  int device = -1;
-  char* host = nullptr;             // pinned; the device uses the same address
-  size_t bytes = 0;
-  hipStream_t stream[2] = {nullptr, nullptr};
-  hipEvent_t done[kEvalSlots] = {nullptr, nullptr, nullptr, nullptr};
-
-  int reserve(size_t want) {
-    if (want <= bytes) return SMA_OK;
-    size_t nb = bytes ? bytes : 4096;
-    while (nb < want) nb *= 2;
-    if (host) (void)hipHostFree(host);
-    host = nullptr;
-    bytes = 0;
-    void* p = nullptr;
-    HIPCHK(hipHostMalloc(&p, nb, hipHostMallocMapped | hipHostMallocCoherent));
-    host = (char*)p;
-    HIPCHK(hipHostGetDevicePointer(&p, host, 0));
-    if (p != host) return fail(SMA_ERR_HIP, "sma160_eval: pinned memory has no common address");
-    bytes = nb;
-    return SMA_OK;
-  }
-  int open(int dev) {
-    device = dev;
-    for (auto& q : stream) HIPCHK(hipStreamCreateWithFlags(&q, hipStreamNonBlocking));
-    for (auto& e : done) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    return SMA_OK;
-  }
-  void close() {
-    for (auto& e : done)
-      if (e) (void)hipEventDestroy(e);
-    for (auto& q : stream)
-      if (q) (void)hipStreamDestroy(q);
-    if (host) (void)hipHostFree(host);
-  }
-};
-std::mutex g_eval_mu;
-EvalStage* g_eval_pool[kEvalPool] = {};
-
-// A stage of the current device, given back (its streams idle) when the
-// call ends.
-class EvalLease {
- public:
-  EvalStage* st = nullptr;
-  bool busy = false;                // kernels or copies may still run
-  int take() {
-    int dev = 0;
-    HIPCHK(hipGetDevice(&dev));
-    {
-      std::lock_guard<std::mutex> lock(g_eval_mu);
-      for (auto& p : g_eval_pool)
-        if (p && p->device == dev) {
-          st = p;
-          p = nullptr;
-          return SMA_OK;
-        }
-    }
-    st = new (std::nothrow) EvalStage();
-    if (!st) return fail(SMA_ERR_HIP, "sma160_eval: out of memory");
-    return st->open(dev);
-  }
-  ~EvalLease() {
-    if (!st) return;
-    if (busy)
-      for (auto& q : st->stream) (void)hipStreamSynchronize(q);
-    if (st->bytes > kEvalKeep) {
-      (void)hipHostFree(st->host);
-      st->host = nullptr;
-      st->bytes = 0;
-    }
-    {
-      std::lock_guard<std::mutex> lock(g_eval_mu);
-      for (auto& p : g_eval_pool)
-        if (!p && st->done[kEvalSlots - 1]) {
-          p = st;
-          return;
-        }
-    }
-    st->close();
-    delete st;
-  }
-};
 
 static int law_launch(int64_t n, int32_t nmat, const double* props, const int32_t* mat, const double* E,
                       const double* F, const double* sdv_old, double* sdv_new, double* S,
@@ -1889,9 +1952,9 @@ int sma160_eval(int64_t n, int32_t n_mat, const double* props, const int32_t* ma
     for (int64_t i = 0; i < n; ++i)
       if (mat_of_gp[i] < 0 || mat_of_gp[i] >= n_mat)
         return fail(SMA_ERR_ARG, "sma160_eval: material index out of range");
-  EvalLease lease;
+  HostLease lease;
   if (int rc = lease.take()) return rc;
-  EvalStage& st = *lease.st;
+  HostStage& st = *lease.st;
   // equal chunks of whole waves; a slot holds a chunk's sections, inputs first.
   // A chunk's outputs are stored before a later chunk's inputs are read: fine
   // for distinct arrays and for a call in place, one chunk for other overlaps.
@@ -1914,7 +1977,7 @@ int sma160_eval(int64_t n, int32_t n_mat, const double* props, const int32_t* ma
   const size_t slot_bytes = (size_t)per * (8 * cols + (mat_of_gp ? 4 : 0) + (flags ? 4 : 0)) + 8;
   const size_t span = (slot_bytes + 255) / 256 * 256, b_props = (size_t)n_mat * 18 * 8;
   const size_t head = (b_props + 255) / 256 * 256;
-  if (int rc = st.reserve(head + span * (size_t)std::min<int64_t>(nchunk, kEvalSlots))) return rc;
+  if (int rc = st.reserve(head + span * (size_t)std::min<int64_t>(nchunk, kStageSlots))) return rc;
   std::memcpy(st.host, props, b_props);
   struct Slot {
     double *F, *so, *E, *sn, *S;
@@ -1923,7 +1986,7 @@ int sma160_eval(int64_t n, int32_t n_mat, const double* props, const int32_t* ma
   };
   auto slot_of = [&](int64_t c) {
     Slot q{};
-    double* d = (double*)(st.host + head + span * (size_t)(c % kEvalSlots));
+    double* d = (double*)(st.host + head + span * (size_t)(c % kStageSlots));
     q.F = d;
     q.so = q.F + 9 * per;
     q.sn = q.so + 3 * per;
@@ -1946,11 +2009,11 @@ int sma160_eval(int64_t n, int32_t n_mat, const double* props, const int32_t* ma
     lease.busy = true;
     if (int rc = law_launch(m, n_mat, (const double*)st.host, q.mat, q.E, q.F, q.so, q.sn, q.S, q.fl, precision, s))
       return rc;
-    if (nchunk > 1) HIPCHK(hipEventRecord(st.done[c % kEvalSlots], s));
+    if (nchunk > 1) HIPCHK(hipEventRecord(st.done[c % kStageSlots], s));
     return SMA_OK;
   };
   auto drain = [&](int64_t c) -> int {
-    if (nchunk > 1) HIPCHK(hipEventSynchronize(st.done[c % kEvalSlots]));
+    if (nchunk > 1) HIPCHK(hipEventSynchronize(st.done[c % kStageSlots]));
     else HIPCHK(hipStreamSynchronize(st.stream[0]));
     const Slot q = slot_of(c);
     const int64_t i0 = c * per, m = std::min(per, n - i0);
@@ -1959,9 +2022,9 @@ int sma160_eval(int64_t n, int32_t n_mat, const double* props, const int32_t* ma
     if (q.fl) std::memcpy(flags + i0, q.fl, (size_t)m * 4);
     return SMA_OK;
   };
-  for (int64_t c = 0; c < nchunk + kEvalSlots; ++c) {
-    if (c >= kEvalSlots && c - kEvalSlots < nchunk)
-      if (int rc = drain(c - kEvalSlots)) return rc;
+  for (int64_t c = 0; c < nchunk + kStageSlots; ++c) {
+    if (c >= kStageSlots && c - kStageSlots < nchunk)
+      if (int rc = drain(c - kStageSlots)) return rc;
     if (c < nchunk)
       if (int rc = fill(c)) return rc;
   }

@@ -1691,6 +1691,33 @@ __global__ void sld_reciprocal(const double* __restrict__ m, double* __restrict_
 }
 
 // ----------------------------------------------------------------------------
+// Read-back: components of a field (one array each) interleaved by rows, with
+// the caller's element order, as the host wants them.  One value a thread, so
+// a wave writes 512 consecutive bytes; the output is pinned host memory, whose
+// link (55 GB/s) is the bound.
+// ----------------------------------------------------------------------------
+struct PackArgs {
+  const void* src[9];
+  int32_t fp32;                 // the sources are float
+  const int32_t* stored;        // rows are Gauss points: stored position of each element, or null
+  int64_t row0, same;           // component 2 of stored rows below `same` is component 1
+  int32_t rows;
+  double* out;                  // [rows][NC]
+};
+
+template <int NC>
+__global__ void __launch_bounds__(256) sld_pack(PackArgs A) {
+  const int j = blockIdx.x * 256 + threadIdx.x;
+  if (j >= A.rows * NC) return;
+  const int r = j / NC;
+  int k = j - r * NC;
+  int64_t i = A.row0 + r;
+  if (A.stored) i = 8 * (int64_t)A.stored[i >> 3] + (i & 7);
+  if (NC == 3 && k == 2 && i < A.same) k = 1;
+  A.out[j] = A.fp32 ? (double)((const float*)A.src[k])[i] : ((const double*)A.src[k])[i];
+}
+
+// ----------------------------------------------------------------------------
 // Point-wise law (drop-in for eval_sld_stress_model_160 with flagt = 0).
 // Bound by memory: 212 bytes a point (F, S, history, E, material, flags).  The
 // stresses, a third of it, are stored past the caches: nothing here reads them

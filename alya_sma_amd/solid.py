@@ -269,7 +269,7 @@ class Solidz:
                      6: ((e, 8, 9), np.float64), 7: ((e, 8), np.uint32), 8: ((1,), np.float64),
                      9: ((8,), np.uint64), 10: ((e, 8, 9), np.float64),
                      11: ((n, 3), np.float64), 12: ((4,), np.float64)}[f]
-        out = np.zeros(shape, dtype=dt)
+        out = np.empty(shape, dtype=dt)
         check(lib().sld_dev_get(self.h, f, _p(out), out.size), f"sld_dev_get({field})")
         return out
 
