@@ -1033,6 +1033,8 @@ int sld_dev_create(const sld_mesh_desc* mesh, const sld_material_desc* mat,
       if (fext_func >= 0 &&
           (bc->fext0[3 * p] != 0.0 || bc->fext0[3 * p + 1] != 0.0 || bc->fext0[3 * p + 2] != 0.0))
         fm[p] |= (uint8_t)sld::FIX_FORCE;
+      if (bc->func_of_node && bc->func_of_node[p] >= 0)
+        fm[p] |= (uint8_t)(std::min(bc->func_of_node[p] + 1, sld::FIX_FUNC_LOOKUP) << sld::FIX_FUNC_SHIFT);
     }
     TRY(upload(&d->fixmask, fm.data(), (size_t)np, s)); track(d, d->fixmask);
   }
