@@ -894,6 +894,15 @@ __device__ inline sma::ReturnMap surrogate_or_exact(const ElemArgs& A, const sma
   return rm;
 }
 
+// The value of x, opaque to the optimiser: quantities derived from the lane
+// index (shape-function derivatives at the lane's Gauss point or node) are
+// then recomputed where they are used instead of being hoisted out of the
+// tile loop and held in registers through the constitutive update.
+__device__ __forceinline__ int opaque(int x) {
+  asm volatile("" : "+v"(x));
+  return x;
+}
+
 // Wave-level flag counters: 64-bit atomics on the wave's counter line, lane 0
 // adding its KF_AS count and lane 1 its KF_SA count in one instruction; the
 // other bits (rare) one by one.
@@ -902,7 +911,7 @@ __device__ __forceinline__ void count_flags(unsigned long long* ctr, uint32_t fl
   if (__ballot(fl != 0u) == 0ull) return;   // wave-uniform: nothing to count
   ctr += 8 * (blockIdx.x % COUNTER_SLOTS);
   static_assert(sma::FLAG_KF_AS == 1u && sma::FLAG_KF_SA == 2u, "counters 0 and 1");
-  const int lane = threadIdx.x & 63;
+  const int lane = opaque(threadIdx.x) & 63;
   const int n0 = __popcll(__ballot(fl & sma::FLAG_KF_AS));
   const int n1 = __popcll(__ballot(fl & sma::FLAG_KF_SA));
   const int n = lane == 0 ? n0 : n1;
@@ -949,18 +958,21 @@ __device__ __forceinline__ void wave_sync() {
 #define SLD_WAVES_F32 4
 #endif
 #ifndef SLD_WAVES_F64_SMA
-#define SLD_WAVES_F64_SMA 4
+#define SLD_WAVES_F64_SMA 5
 #endif
 // LAWS = 0: each element takes its own law (law_of_elem); LAWS = 1: every
 // element of the launch is SMA (a mesh without neo-Hookean elements, or the
 // SMA range of a law-grouped mesh), without the neo-Hookean path, whose
-// registers would otherwise add to the SMA path's (FP64: 126 VGPRs and 4
-// waves per SIMD against 167 and 3); LAWS = 2: every element of the launch
-// is neo-Hookean (the tissue range of a law-grouped mesh), without the SMA
-// path (FP64: 108 VGPRs; FP32: 56, 8 waves).  FP64 and FP32 SMA kernels at 5
-// waves per SIMD spill 10 registers and run slower (C1: 44.6 against 40.4 us
-// and 30.5 against 28.9).  Kernels that also store the stresses (STORE) keep 3
-// waves in FP64 and 6 in the FP32 neo-Hookean kernel.
+// registers would otherwise add to the SMA path's; LAWS = 2: every element of
+// the launch is neo-Hookean (the tissue range of a law-grouped mesh), without
+// the SMA path (FP64: 72 VGPRs, 7 waves per SIMD; FP32: 56, 8).  The FP64 SMA
+// kernel needs 94 VGPRs (5 waves) since nothing of the rarely taken branches
+// is held through it: constants of long series and of library functions were
+// 32 of its 126 registers (4 waves) and 40 of its ~800 instructions.  C1 38.6
+// -> 35.5 us, 64 specimens 158 -> 154.5, tube 117 -> 113; 3 waves: 40 and 178,
+// and with 5 registers spilled at 5 waves 38 and 182.  FP32 SMA kernels stay
+// at 4 waves (5 spill and are slower).  Kernels that also store the stresses
+// (STORE) keep 3 waves in FP64 and 6 in the FP32 neo-Hookean kernel.
 template <typename R, int LAWS = 0, bool DAMP = false, bool STORE = false>
 struct ElemOccupancy {
   static constexpr int waves = DAMP ? (sizeof(R) == 8 ? 1 : 2)
@@ -990,15 +1002,6 @@ __device__ __forceinline__ R sign_if(R c, int neg) {
     return __longlong_as_double(__double_as_longlong(c) ^ ((long long)(neg & 1) << 63));
   else
     return __int_as_float(__float_as_int(c) ^ (int)((unsigned)(neg & 1) << 31));
-}
-
-// The value of x, opaque to the optimiser: quantities derived from the lane
-// index (shape-function derivatives at the lane's Gauss point or node) are
-// then recomputed where they are used instead of being hoisted out of the
-// tile loop and held in registers through the constitutive update.
-__device__ __forceinline__ int opaque(int x) {
-  asm volatile("" : "+v"(x));
-  return x;
 }
 
 // DAMP: Rayleigh damping (sld_elmmat.f90:160-163, :174-194) -- the

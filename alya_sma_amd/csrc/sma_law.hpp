@@ -131,22 +131,26 @@ __host__ __device__ __forceinline__ double rcp64(double x) {
 // sqrt(s) and 1/sqrt(s) of s >= 0 together: the hardware estimate refined by
 // two Newton steps (1 ulp), the root corrected once more by its residual;
 // 12 instructions against ~25 for an IEEE root and a division by it.  Below
-// 1e-290 (where the refinement would lose digits) the root is the library's
-// and its reciprocal 0 for s = 0.
+// 1e-290 (where the refinement would lose digits) s is scaled first; the
+// reciprocal of 0 is 0.
 __host__ __device__ __forceinline__ void sqrt_rsqrt64(double s, double& root, double& inv) {
+  const bool small = !(s >= 1e-290);
+  double t = s;
+  if (small) t = s * 0x1p600;
 #if defined(__HIP_DEVICE_COMPILE__)
-  if (s >= 1e-290) {
-    double y = __builtin_amdgcn_rsq(s);
-    y = fma(0.5 * y, fma(-s * y, y, 1.0), y);
-    y = fma(0.5 * y, fma(-s * y, y, 1.0), y);
-    const double r = s * y;
-    root = fma(fma(-r, r, s), 0.5 * y, r);
-    inv = y;
-    return;
-  }
+  double y = __builtin_amdgcn_rsq(t);
+#else
+  double y = 1.0 / sqrt(t);
 #endif
-  root = sqrt(s);
-  inv = root > 0.0 ? 1.0 / root : 0.0;
+  y = fma(0.5 * y, fma(-t * y, y, 1.0), y);
+  y = fma(0.5 * y, fma(-t * y, y, 1.0), y);
+  const double r = t * y;
+  root = fma(fma(-r, r, t), 0.5 * y, r);
+  inv = y;
+  if (small) {
+    root = s == 0.0 ? 0.0 : root * 0x1p-300;
+    inv = s > 0.0 ? y * 0x1p300 : 0.0;
+  }
 }
 
 // J^(-2/3) in FP64 (the neo-Hookean law's volumetric factor).  On the
@@ -154,22 +158,34 @@ __host__ __device__ __forceinline__ void sqrt_rsqrt64(double s, double& root, do
 // (relative error ~3e-7), refined by two Newton steps on y^-3 = J,
 // y <- y + y (1 - J y^3) / 3 (error e -> -2 e^2: 3e-7 -> 2e-13 -> rounding),
 // then squared: within 2 ulps of the exact value (pow: 1), in ~20
-// instructions against pow's ~170.  J outside [2^-100, 2^100], NaN
-// included, takes pow.
+// instructions against pow's ~170.  J outside [2^-100, 2^100] is first scaled
+// by a power of 8 and the result by the power of 4 (both exact); a J that is
+// not positive and finite gives what pow gives.  (A call of pow there put its
+// 38 constants into vector registers at the start of every wave: 6% of the
+// neo-Hookean element kernel's instructions, 28 of its 108 registers.)
 __host__ __device__ __forceinline__ double pow_m23(double J) {
+  int k = 0;
+  if (!(J >= 0x1p-100 && J <= 0x1p100)) {
+    if (!(J > 0.0 && J < __builtin_inf()))
+      return J == 0.0 ? __builtin_inf() : J == __builtin_inf() ? 0.0 : __builtin_nan("");
 #if defined(__HIP_DEVICE_COMPILE__)
-  if (!(J >= 0x1p-100 && J <= 0x1p100)) return pow(J, -2.0 / 3.0);
-  const float l2 = __builtin_amdgcn_logf((float)J);
-  double y = (double)__builtin_amdgcn_exp2f(l2 * (-1.0f / 3.0f));
+    k = __builtin_amdgcn_frexp_exp(J) / 3;
+#else
+    k = (ilogb(J) + 1) / 3;
+#endif
+    J = ldexp(J, -3 * k);
+  }
+#if defined(__HIP_DEVICE_COMPILE__)
+  double y = (double)__builtin_amdgcn_exp2f(__builtin_amdgcn_logf((float)J) * (-1.0f / 3.0f));
+#else
+  double y = (double)exp2f(log2f((float)J) * (-1.0f / 3.0f));
+#endif
 #pragma unroll
-  for (int k = 0; k < 2; ++k) {
+  for (int n = 0; n < 2; ++n) {
     const double r = fma(-J * y, y * y, 1.0);
     y = fma(y * (1.0 / 3.0), r, y);
   }
-  return y * y;
-#else
-  return pow(J, -2.0 / 3.0);
-#endif
+  return ldexp(y * y, -2 * k);
 }
 
 // One Givens step of the implicit-shift QL sweep (dsyevq3.f90:99-129) on
@@ -555,7 +571,7 @@ __host__ __device__ __forceinline__ void cayley(const R (&c)[6], R (&z)[6]) {
           a4 = c[1] * c[2] - c[0] * c[4], a5 = c[0] * c[3] - c[1] * c[1];
   const R i2 = a0 + a3 + a5, i3 = c[0] * a0 + c[1] * a1 + c[2] * a2;
   const R q = R(2) * i2 + i3;
-  const R r = rcp_r<R>(R(8) + R(4) * (c[0] + c[3] + c[5]) + q);
+  const R r = rcp_r<R>(R(4) * (R(2) + (c[0] + c[3] + c[5])) + q);
   z[0] = (R(4) * c[0] + (q - R(2) * a0)) * r;
   z[1] = (R(4) * c[1] - R(2) * a1) * r;
   z[2] = (R(4) * c[2] - R(2) * a2) * r;
@@ -711,22 +727,33 @@ struct HenckyTerms {
 constexpr double kTerms3 = 1.4949e-04, kTerms4 = 9.0589e-04, kTerms5 = 2.9934e-03,
                  kTerms6 = 7.0039e-03, kTerms7 = 1.3216e-02, kTerms8 = 2.1619e-02,
                  kTerms10 = 4.4078e-02, kTerms15 = 1.1898e-01, kTerms22 = 2.2961e-01;
+// 1/N, formed where it is used: the empty asm keeps the compiler from holding
+// the coefficients of all series lengths in vector registers from the start of
+// a wave (34 instructions of ~800 and 26 of 126 registers of the element kernel).
+template <int N>
+__host__ __device__ __forceinline__ double odd64() {
+  double c = 1.0 / N;
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("" : "+s"(c));
+#endif
+  return c;
+}
 __host__ __device__ __forceinline__ HenckyTerms hencky64_terms(double zf2) {
   const bool m3 = zf2 > kTerms3;
-  if (!any_lane(m3)) return {3, 1.0 / 5, 1.0 / 7};
+  if (!any_lane(m3)) return {3, odd64<5>(), odd64<7>()};
   const bool m4 = zf2 > kTerms4;
-  if (!any_lane(m4)) return {4, 1.0 / 7, m3 ? 1.0 / 9 : 0.0};
+  if (!any_lane(m4)) return {4, odd64<7>(), m3 ? odd64<9>() : 0.0};
   const bool m5 = zf2 > kTerms5;
-  if (!any_lane(m5)) return {5, m3 ? 1.0 / 9 : 0.0, m4 ? 1.0 / 11 : 0.0};
+  if (!any_lane(m5)) return {5, m3 ? odd64<9>() : 0.0, m4 ? odd64<11>() : 0.0};
   const bool m6 = zf2 > kTerms6;
-  if (!any_lane(m6)) return {6, m4 ? 1.0 / 11 : 0.0, m5 ? 1.0 / 13 : 0.0};
+  if (!any_lane(m6)) return {6, m4 ? odd64<11>() : 0.0, m5 ? odd64<13>() : 0.0};
   const bool m7 = zf2 > kTerms7;
-  if (!any_lane(m7)) return {7, m5 ? 1.0 / 13 : 0.0, m6 ? 1.0 / 15 : 0.0};
-  if (!any_lane(zf2 > kTerms8)) return {8, m6 ? 1.0 / 15 : 0.0, m7 ? 1.0 / 17 : 0.0};
-  if (!any_lane(zf2 > kTerms10)) return {10, zf2 > kTerms8 ? 1.0 / 19 : 0.0, zf2 > kTerms8 ? 1.0 / 21 : 0.0};
-  if (!any_lane(zf2 > kTerms15)) return {15, zf2 > kTerms10 ? 1.0 / 29 : 0.0, zf2 > kTerms10 ? 1.0 / 31 : 0.0};
-  if (!any_lane(zf2 > kTerms22)) return {22, zf2 > kTerms15 ? 1.0 / 43 : 0.0, zf2 > kTerms15 ? 1.0 / 45 : 0.0};
-  return {32, zf2 > kTerms22 ? 1.0 / 63 : 0.0, zf2 > kTerms22 ? 1.0 / 65 : 0.0};   // zf2 <= 0.36
+  if (!any_lane(m7)) return {7, m5 ? odd64<13>() : 0.0, m6 ? odd64<15>() : 0.0};
+  if (!any_lane(zf2 > kTerms8)) return {8, m6 ? odd64<15>() : 0.0, m7 ? odd64<17>() : 0.0};
+  if (!any_lane(zf2 > kTerms10)) return {10, zf2 > kTerms8 ? odd64<19>() : 0.0, zf2 > kTerms8 ? odd64<21>() : 0.0};
+  if (!any_lane(zf2 > kTerms15)) return {15, zf2 > kTerms10 ? odd64<29>() : 0.0, zf2 > kTerms10 ? odd64<31>() : 0.0};
+  if (!any_lane(zf2 > kTerms22)) return {22, zf2 > kTerms15 ? odd64<43>() : 0.0, zf2 > kTerms15 ? odd64<45>() : 0.0};
+  return {32, zf2 > kTerms22 ? odd64<63>() : 0.0, zf2 > kTerms22 ? odd64<65>() : 0.0};   // zf2 <= 0.36
 }
 // 1/(2k+1), k = 7..30: the coefficients of the long series
 constexpr double kInvOdd64[24] = {
@@ -773,12 +800,12 @@ __host__ __device__ __forceinline__ Hencky64 hencky_fp64(const double (&H)[9]) {
                  : zf2 > kTerms8 ? 10 : zf2 > kTerms7 ? 8 : zf2 > kTerms6 ? 7 : 6;
     for (int k = n - 2; k > 6; --k) r.step(k <= nl ? kInvOdd64[k - 7] : 0.0);
   }
-  if (n > 7) r.step(zf2 > kTerms5 ? 1.0 / 13.0 : 0.0);   // k = 6
-  if (n > 6) r.step(zf2 > kTerms4 ? 1.0 / 11.0 : 0.0);
-  if (n > 5) r.step(zf2 > kTerms3 ? 1.0 / 9.0 : 0.0);
-  if (n > 4) r.step(1.0 / 7.0);
-  if (n > 3) r.step(1.0 / 5.0);
-  r.step(1.0 / 3.0);                                     // k = 1
+  if (n > 7) r.step(zf2 > kTerms5 ? odd64<13>() : 0.0);   // k = 6
+  if (n > 6) r.step(zf2 > kTerms4 ? odd64<11>() : 0.0);
+  if (n > 5) r.step(zf2 > kTerms3 ? odd64<9>() : 0.0);
+  if (n > 4) r.step(odd64<7>());
+  if (n > 3) r.step(odd64<5>());
+  r.step(1.0 / 3.0);                                      // k = 1
   r.step(1.0);
   double en2;
   r.strain(z, w, zf2, (double)(1 << halvings), h.theta, h.ed, en2);
@@ -932,6 +959,9 @@ __host__ __device__ __forceinline__ bool return_map_closed(const Mat& m, double 
   return done;
 }
 
+// The largest q whose square root, rounded, is at most 1.0e-8: sqrt(q) > 1.0e-8
+// is q > kResi2.
+constexpr double kResi2 = 0x1.cd2b297d889bdp-54;
 __host__ __device__ __forceinline__ ReturnMap return_map(const Mat& m, double theta, double e_n,
                                                 double xS_0, double F_AS_0, double F_SA_0) {
 #pragma clang fp contract(off)
@@ -944,9 +974,9 @@ __host__ __device__ __forceinline__ ReturnMap return_map(const Mat& m, double th
   double dh_AS = 0.0, dh_SA = 0.0;
   double RHS_AS = (F_AS - m.Rf_AS) * dh_AS + H_AS * F_AS_dot * (1.0 - xS);
   double RHS_SA = (F_SA - m.Rf_SA) * dh_SA - H_SA * F_SA_dot * xS;
-  double resi = RHS_AS * RHS_AS + RHS_SA * RHS_SA;   // squared first (:403)
+  bool more = RHS_AS * RHS_AS + RHS_SA * RHS_SA > 1.0e-8;   // squared first (:403)
   int iter = 0;
-  while (iter < 65 && resi > 1.0e-8) {
+  while (iter < 65 && more) {
     ++iter;
     double m11 = -m.G_1 * dh_AS - (H_AS * F_AS_dot + H_AS * (1.0 - xS) * m.G_1) + (F_AS - m.Rf_AS);
     double m12 = -m.G_1 * dh_AS - (H_AS * F_AS_dot + H_AS * (1.0 - xS) * m.G_1);
@@ -965,7 +995,7 @@ __host__ __device__ __forceinline__ ReturnMap return_map(const Mat& m, double th
     F_SA_dot = F_SA - F_SA_0;
     RHS_AS = (F_AS - m.Rf_AS) * dh_AS + H_AS * F_AS_dot * (1.0 - xS);
     RHS_SA = (F_SA - m.Rf_SA) * dh_SA - H_SA * F_SA_dot * xS;
-    resi = sqrt(RHS_AS * RHS_AS + RHS_SA * RHS_SA);
+    more = RHS_AS * RHS_AS + RHS_SA * RHS_SA > kResi2;
   }
   if (iter >= 65) {                                  // revert (:459-465)
     r.flags |= FLAG_NEWTON_FAIL;
