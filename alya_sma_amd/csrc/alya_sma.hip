@@ -303,6 +303,13 @@ void launch_element(sld::ElemArgs A, hipStream_t s, int persistent) {
       grid = (ntiles + A.tiles_per_block - 1) / A.tiles_per_block;
     }
   }
+  if constexpr (sizeof(R) == 8 && EPB == 8 && !STORE && SUR == 0 && GATHER && LAWS == 1 && !DAMP) {
+    if (A.one_f) {
+      hipLaunchKernelGGL((sld::sld_element<R, EPB, STORE, SUR, GATHER, LAWS, DAMP, true>), dim3(grid),
+                         dim3(EPB * 8), 0, s, A);
+      return;
+    }
+  }
   hipLaunchKernelGGL((sld::sld_element<R, EPB, STORE, SUR, GATHER, LAWS, DAMP>), dim3(grid),
                      dim3(EPB * 8), 0, s, A);
 }
@@ -489,6 +496,7 @@ int enqueue_step(sld_dev* d, double dt, int scheme, double phi, int tn, KernelTi
     if (d->one_f) {
       E.sdv_n[2] = E.sdv_n[1];
       E.sdv_k[2] = E.sdv_k[1];
+      E.one_f = 1;
     }
     E.efor = d->efor;
     E.corner_slot = d->corner_slot;
