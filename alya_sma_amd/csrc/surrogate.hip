@@ -183,7 +183,7 @@ int sma_mlp_forward_device(sma_mlp* m, int64_t n, const float* X, float* Y, void
                              (int)mlp::INF_SMEM));
     attr = true;
   }
-  const int64_t nblk = (n + mlp::INF_ROWS - 1) / mlp::INF_ROWS;
+  const int64_t nblk = (n + 15) / 16;   // the smallest row blocks
   int dev = 0, ncu = 256;
   (void)hipGetDevice(&dev);
   (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
@@ -264,7 +264,7 @@ int sma_mlp_infer_listed(sma_mlp* m, const float* X, const unsigned* seg_count, 
   (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
   const int64_t cap = seg_cap * mlp::LIST_SEGS;
   const unsigned grid =
-      (unsigned)std::max<int64_t>(1, std::min<int64_t>((cap + mlp::INF_ROWS - 1) / mlp::INF_ROWS, ncu));
+      (unsigned)std::max<int64_t>(1, std::min<int64_t>((cap + 15) / 16, ncu));
   hipLaunchKernelGGL(mlp::mlp_infer, dim3(grid), dim3(mlp::INF_THREADS), mlp::INF_SMEM, s, m->Wi, m->bp, X,
                      (int64_t)0, seg_count, seg_cap, Y);
   SCHK(hipGetLastError());

@@ -528,9 +528,15 @@ __global__ void pack_params(const float* __restrict__ W, const float* __restrict
 // A wave carries two 16-row blocks (each A fragment read from LDS feeds two
 // MFMA) in 228 VGPRs, so the workgroup has 8 waves, two per SIMD: one
 // wave's SiLU epilogue (two quarter-rate transcendentals per activation,
-// the kernel's largest cost) overlaps the other's MFMA.  Waves take 32-row
-// blocks round robin over the grid (block k on workgroup k mod grid), so a
-// short list spreads over every CU.
+// the kernel's largest cost) overlaps the other's MFMA.  What bounds it: those, 44
+// cycles an activation, 30 us of VALU time for 200 000 rows (their products take
+// 9 of the matrix cores').  Waves take 32-row blocks round robin over the grid
+// (block k on workgroup k mod grid), so a short list spreads over every CU; the
+// rows left after the full rounds go by 16 to a wave when that takes them all,
+// since a wave with a lone 32-row block at the end runs half a round longer.
+// Rows, before -> with 16-row ends: 500 10.4 -> 7.8 us, 16384 11.1 -> 8.7,
+// 200000 44.9 -> 41.5, 400000 80 -> 78; the same where the rest is more than half
+// a round (40000: 15.8).
 // ----------------------------------------------------------------------------
 constexpr int INF_WAVES = 8;
 constexpr int INF_THREADS = INF_WAVES * 64;
@@ -543,21 +549,23 @@ __device__ __forceinline__ bf16x8 cat4(bf16x4 a, bf16x4 b) {
 // A layer's accumulators start at its bias (lane (r, q) holds features
 // 16 b + 4 q + i), so the MFMA chain leaves Z = W x + b and the epilogue
 // adds nothing
-__device__ __forceinline__ void bias_init(f32x4 (&acc)[INF_RB][8], const float* bias, int q) {
+template <int RB>
+__device__ __forceinline__ void bias_init(f32x4 (&acc)[RB][8], const float* bias, int q) {
 #pragma unroll
   for (int b = 0; b < 8; ++b) {
     const f32x4 bc = *reinterpret_cast<const f32x4*>(bias + 16 * b + 4 * q);
 #pragma unroll
-    for (int a = 0; a < INF_RB; ++a) acc[a][b] = bc;
+    for (int a = 0; a < RB; ++a) acc[a][b] = bc;
   }
 }
 
 // SiLU of one layer's Z into the next layer's inputs
-__device__ __forceinline__ void hidden_epilogue(const f32x4 (&acc)[INF_RB][8], bf16x4 (&h)[INF_RB][8]) {
+template <int RB>
+__device__ __forceinline__ void hidden_epilogue(const f32x4 (&acc)[RB][8], bf16x4 (&h)[RB][8]) {
 #pragma unroll
   for (int b = 0; b < 8; ++b)
 #pragma unroll
-    for (int a = 0; a < INF_RB; ++a)
+    for (int a = 0; a < RB; ++a)
 #pragma unroll
       for (int i = 0; i < 4; ++i) h[a][b][i] = (__bf16)silu(acc[a][b][i]);
 }
@@ -572,9 +580,13 @@ __global__ void __launch_bounds__(INF_THREADS) mlp_infer(const __bf16* __restric
   // point's row is its slot
   __shared__ unsigned off[LIST_SEGS + 1];
   const int64_t n = seg_count ? (int64_t)list_scan(seg_count, off) : n_host;
-  const int64_t nblk = (n + INF_ROWS - 1) / INF_ROWS;
+  // full rounds of INF_ROWS rows for every wave, then the rest: 16 rows a wave
+  // if that takes them all, so that a last round costs half a block's time
+  const int64_t nwaves = (int64_t)gridDim.x * INF_WAVES;
+  const int64_t full = n / (nwaves * INF_ROWS), rest0 = full * nwaves * INF_ROWS, rest = n - rest0;
+  const int rest_rows = rest > 16 * nwaves ? INF_ROWS : 16;
   // a workgroup without a row block leaves before copying the weights
-  if ((int64_t)blockIdx.x >= nblk) return;
+  if (full == 0 && (int64_t)blockIdx.x * rest_rows >= rest) return;
   extern __shared__ __align__(16) unsigned char smem[];
   __bf16* sW = reinterpret_cast<__bf16*>(smem);
   float* sb = reinterpret_cast<float*>(smem + WLDS_TOTAL * sizeof(__bf16));
@@ -587,19 +599,19 @@ __global__ void __launch_bounds__(INF_THREADS) mlp_infer(const __bf16* __restric
   __syncthreads();
   const int lane = tid & 63, wave = tid >> 6;
   const int r = lane & 15, q = lane >> 4;
-  const int64_t nwaves = (int64_t)gridDim.x * INF_WAVES;
   static_assert(INF_ROWS <= 64, "one lane holds the slot of each row of a block");
-  for (int64_t blk = (int64_t)wave * gridDim.x + blockIdx.x; blk < nblk; blk += nwaves) {
-    const int64_t row0 = blk * INF_ROWS;
-    // lane l < INF_ROWS: the slot of row row0 + l
+  // RB 16-row blocks from row0 on
+  auto block = [&](auto rb, int64_t row0) {
+    constexpr int RB = decltype(rb)::value;
+    // lane l < 16 RB: the slot of row row0 + l
     int slot_l = 0;
-    if (lane < INF_ROWS && row0 + lane < n)
+    if (lane < 16 * RB && row0 + lane < n)
       slot_l = seg_count ? (int)list_slot(off, (unsigned)(row0 + lane), seg_cap) : (int)(row0 + lane);
     // layer 0's B fragments: inputs 8 q .. 8 q + 7 of row 16 a + r (NIN = 16
     // real inputs; lanes q >= 2 hold the zero padding)
-    bf16x8 x0[INF_RB];
+    bf16x8 x0[RB];
 #pragma unroll
-    for (int a = 0; a < INF_RB; ++a) {
+    for (int a = 0; a < RB; ++a) {
       const int64_t sl = __shfl(slot_l, 16 * a + r);
       float4 lo = make_float4(0.f, 0.f, 0.f, 0.f), hi = lo;
       if (q < 2 && row0 + 16 * a + r < n) {
@@ -610,15 +622,15 @@ __global__ void __launch_bounds__(INF_THREADS) mlp_infer(const __bf16* __restric
       x0[a] = bf16x8{(__bf16)lo.x, (__bf16)lo.y, (__bf16)lo.z, (__bf16)lo.w,
                      (__bf16)hi.x, (__bf16)hi.y, (__bf16)hi.z, (__bf16)hi.w};
     }
-    bf16x4 h[INF_RB][8];
-    f32x4 acc[INF_RB][8];
+    bf16x4 h[RB][8];
+    f32x4 acc[RB][8];
     // layer 0 (K = 32)
     bias_init(acc, sb + boff(0), q);
 #pragma unroll
     for (int b = 0; b < 8; ++b) {
       const bf16x8 wf = *reinterpret_cast<const bf16x8*>(sW + (16 * b + r) * wld(0) + 8 * q);
 #pragma unroll
-      for (int a = 0; a < INF_RB; ++a)
+      for (int a = 0; a < RB; ++a)
         acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, x0[a], acc[a][b], 0, 0, 0);
     }
     hidden_epilogue(acc, h);
@@ -629,15 +641,15 @@ __global__ void __launch_bounds__(INF_THREADS) mlp_infer(const __bf16* __restric
       bias_init(acc, sb + boff(l), q);
 #pragma unroll
       for (int c = 0; c < NH / 32; ++c) {
-        bf16x8 xf[INF_RB];
+        bf16x8 xf[RB];
 #pragma unroll
-        for (int a = 0; a < INF_RB; ++a) xf[a] = cat4(h[a][2 * c], h[a][2 * c + 1]);
+        for (int a = 0; a < RB; ++a) xf[a] = cat4(h[a][2 * c], h[a][2 * c + 1]);
 #pragma unroll
         for (int b = 0; b < 8; ++b) {
           const bf16x8 wf =
               *reinterpret_cast<const bf16x8*>(W + (16 * b + r) * wld(1) + 32 * c + 8 * q);
 #pragma unroll
-          for (int a = 0; a < INF_RB; ++a)
+          for (int a = 0; a < RB; ++a)
             acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, xf[a], acc[a][b], 0, 0, 0);
         }
       }
@@ -650,19 +662,19 @@ __global__ void __launch_bounds__(INF_THREADS) mlp_infer(const __bf16* __restric
       // features 4 q .. 4 q + 3 of the output block, from its bias (zero
       // beyond NOUT)
       const f32x4 bo = *reinterpret_cast<const f32x4*>(sb + boff(l) + 4 * q);
-      f32x4 o[INF_RB];
+      f32x4 o[RB];
 #pragma unroll
-      for (int a = 0; a < INF_RB; ++a) o[a] = bo;
+      for (int a = 0; a < RB; ++a) o[a] = bo;
 #pragma unroll
       for (int c = 0; c < NH / 32; ++c) {
         const bf16x8 wf = *reinterpret_cast<const bf16x8*>(W + r * wld(l) + 32 * c + 8 * q);
 #pragma unroll
-        for (int a = 0; a < INF_RB; ++a)
+        for (int a = 0; a < RB; ++a)
           o[a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, cat4(h[a][2 * c], h[a][2 * c + 1]),
                                                          o[a], 0, 0, 0);
       }
 #pragma unroll
-      for (int a = 0; a < INF_RB; ++a) {
+      for (int a = 0; a < RB; ++a) {
         const int64_t m = row0 + 16 * a + r;
         const int64_t sl = __shfl(slot_l, 16 * a + r);
 #pragma unroll
@@ -672,6 +684,12 @@ __global__ void __launch_bounds__(INF_THREADS) mlp_infer(const __bf16* __restric
         }
       }
     }
+  };
+  const int64_t wid = (int64_t)wave * gridDim.x + blockIdx.x;
+  for (int64_t k = 0; k < full; ++k) block(std::integral_constant<int, INF_RB>{}, (k * nwaves + wid) * INF_ROWS);
+  if (wid * rest_rows < rest) {
+    if (rest_rows == INF_ROWS) block(std::integral_constant<int, INF_RB>{}, rest0 + wid * INF_ROWS);
+    else block(std::integral_constant<int, 1>{}, rest0 + wid * 16);
   }
 }
 

@@ -51,6 +51,21 @@ def test_forward_large_batch_matches_oracle(sur):
     np.testing.assert_array_equal(Ys, Yg[-77:])
 
 
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 4095, 4097, 32768, 32769, 65535, 65536, 65537, 98304, 98305])
+def test_forward_at_the_ends_of_rounds(sur, n):
+    """Rows left after full rounds (65536 rows on 256 CUs) go by 16 or 32 to a
+    wave: at every border a row's output is the one it has in another batch."""
+    print(f"mlp forward, {n} rows", flush=True)
+    X = np.random.default_rng(7).normal(size=(140000, 16)).astype(np.float32)
+    want = sur.forward(DeviceArray.from_host(X)).to_host()
+    W, b = sur.get_params()
+    Yo, _ = M.forward(W, b, X[:200], emulate=True)
+    assert _rel(want[:200], Yo) < 5e-3
+    for first in (0, 140000 - n):
+        Y = sur.forward(DeviceArray.from_host(X[first:first + n])).to_host()
+        np.testing.assert_array_equal(Y, want[first:first + n])
+
+
 def test_gradient_matches_oracle(sur):
     print("mlp gradient vs oracle", flush=True)
     rng = np.random.default_rng(1)
