@@ -1094,10 +1094,11 @@ __host__ __device__ __forceinline__ void kirchhoff(const Mat& m, const Spectral<
 // reference operation by operation, stays where the series does not reach
 // (stretches beyond about 1/2..2, non-finite or singular F), for deviatoric
 // strains up to 1e-5 (there its own rounding, 1e-16, is seen in the direction
-// e'/|e'| and so in the stress of a transformed point), and where the return
-// map needs the reference's iteration, whose count and end can hang on the last
-// bit.
-constexpr double kSeriesMinEn = 1.0e-5;
+// e'/|e'| and so in the stress of a transformed point), where the return map
+// needs the reference's iteration, whose count and end can hang on the last
+// bit, and where an off-diagonal of b is so small (1e-162 .. 1e-77 beside any
+// stretch) that the reference's Householder step underflows: its NaN is kept.
+constexpr double kSeriesMinEn = 1.0e-5, kSeriesMinB = 1.0e-60;
 __host__ __device__ __forceinline__ ReturnMap law_point(const Mat& m, const double (&F)[9], double xS_0,
                                                         double F_AS_0, double F_SA_0, double (&tau)[6]) {
   ReturnMap rm;
@@ -1105,7 +1106,11 @@ __host__ __device__ __forceinline__ ReturnMap law_point(const Mat& m, const doub
   {
     const double H[9] = {F[0] - 1.0, F[1], F[2], F[3], F[4] - 1.0, F[5], F[6], F[7], F[8] - 1.0};
     const Hencky64 h = hencky_fp64<false>(H);
-    if (h.ok && h.e_n > kSeriesMinEn) {
+    auto tiny = [](double x) { return x != 0.0 && fabs(x) < kSeriesMinB; };
+    const bool under = tiny(F[0] * F[1] + F[3] * F[4] + F[6] * F[7]) ||
+                       tiny(F[0] * F[2] + F[3] * F[5] + F[6] * F[8]) ||
+                       tiny(F[1] * F[2] + F[4] * F[5] + F[7] * F[8]);
+    if (h.ok && h.e_n > kSeriesMinEn && !under) {
       done = return_map_closed(m, h.theta, h.e_n, xS_0, F_AS_0, F_SA_0, rm);
       kirchhoff_hencky64(m, h, rm.xS, tau);
     }

@@ -156,3 +156,17 @@ def test_special_deformations(prog):
         a, b = prog(P, F, np.tile(np.array(sdv, float), (n, 1)))
         # deviatoric strains of rounding size take the spectral form: the same bits
         np.testing.assert_array_equal(a, b)
+
+
+def test_underflow_band_keeps_the_references_answer(prog):
+    """Shear strains whose fourth powers underflow in the reference's
+    Householder step: its NaN, where it gives one, bit for bit otherwise."""
+    tiny = 10.0 ** np.arange(-200, -68, 1.5)
+    F = np.tile(np.diag([1.02, 0.995, 0.99]), (3 * len(tiny), 1, 1))
+    for k, (i, j) in enumerate(((0, 1), (0, 2), (1, 2))):
+        F[k * len(tiny):(k + 1) * len(tiny), i, j] = tiny
+    n = len(F)
+    P = np.tile(NITINOL, (n, 1))
+    a, b = prog(P, F, np.tile([0.0, 0.0, 0.0], (n, 1)))
+    assert np.isnan(b).any()
+    np.testing.assert_array_equal(a, b)
