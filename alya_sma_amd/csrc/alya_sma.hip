@@ -2046,7 +2046,7 @@ int sma160_eval(int64_t n, int32_t n_mat, const double* props, const int32_t* ma
 
 // ---------------------------------------------------------------------------
 // sma160_eval without device allocation.  sma160_eval stages the caller's
-// host arrays through device buffers it allocates and frees on every call;
+// host arrays through pinned blocks of a pool that grows with the calls;
 // sma160_eval_noalloc stages them through `scratch`, a fixed array in the
 // library's device memory.  Being a file-scope __device__ object, every GPU
 // the library runs on holds its own copy (at its own address) until the

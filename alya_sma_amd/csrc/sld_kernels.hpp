@@ -936,10 +936,10 @@ __device__ __forceinline__ void wave_sync() {
 }
 
 // EPB elements per block, 8 threads (one per Gauss point) per element.
-// What bounds it: VALU issue, 75% of the cycles at ~2.05 GHz (C1, FP64: ~750
-// instructions a wave, 3 of 4 in FP64), the rest the first loads of a wave and
-// the launch's start and end.  In FP64 an element's lanes exchange values by
-// DPP moves (hex_grad, hex_grad_t) instead of through LDS: with Walsh-Hadamard
+// What bounds it: VALU issue, 87% of the busy cycles in FP64 at ~2.05 GHz (C1:
+// 663 instructions a wave, 3 of 4 in FP64) and 99% in FP32 (675); the rest the
+// first loads of a wave and the launch's start and end.  In FP64 an element's
+// lanes exchange values by DPP moves (hex_grad, hex_grad_t) instead of through LDS: with Walsh-Hadamard
 // sums and Gauss-point rows in LDS (175 FP64 values read or written per lane)
 // the LDS of a CU, shared by its four SIMDs, was as busy as the VALU, and the
 // two overlapped poorly.  FP64 element launch, before -> with exchanges: C1
@@ -966,7 +966,7 @@ __device__ __forceinline__ void wave_sync() {
 // SMA range of a law-grouped mesh), without the neo-Hookean path, whose
 // registers would otherwise add to the SMA path's; LAWS = 2: every element of
 // the launch is neo-Hookean (the tissue range of a law-grouped mesh), without
-// the SMA path (FP64: 72 VGPRs, 7 waves per SIMD; FP32: 56, 8).  The FP64 SMA
+// the SMA path (FP64: 72 VGPRs, 7 waves per SIMD; FP32: 63, 8).  The FP64 SMA
 // kernel needs 94 VGPRs (5 waves) since nothing of the rarely taken branches
 // is held through it: constants of long series and of library functions were
 // 32 of its 126 registers (4 waves) and 40 of its ~800 instructions.  C1 38.6

@@ -5,9 +5,11 @@
 // INV2x2 :558-573), dsyevq3.f90:22-137 + dsytrd3.f90:22-109 (Kopp's
 // Householder + QL), eigsrt.f90:19-48 (descending selection sort).
 //
-// Two spectral front ends feed one FP64 return map:
+// The strain comes from the series artanh(Z) (hencky_fp64, hencky_fp32) where it
+// reaches, else from one of two spectral front ends; all feed one FP64 return
+// map:
 //   * spectral_fp64: b = F F^T, Kopp QL on b, sqrt/pow/log exactly as the
-//     reference sequences them (plain FP64 mode, parity <= 1e-10);
+//     reference sequences them (point-wise law, parity <= 1e-10);
 //   * spectral_fp32: the same QL on b - I = H + H^T + H H^T (H = F - I) in
 //     FP32, with e_i = log1p(mu_i)/2 - theta/3.  Working on b - I keeps the
 //     small strains at full FP32 relative precision (FP32 kinematics mode).

@@ -73,8 +73,8 @@ int sma160_eval_device(int64_t n_gp, int32_t n_mat, const double *props,
 /* Same arguments and results as sma160_eval (host pointers, synchronous,
  * null stream), with no device allocation: the arrays are staged through a
  * fixed array in the library's device memory (3.4 MB on each GPU it runs
- * on, held until the process ends) instead of buffers allocated and freed
- * per call.  No counterpart in the reference: it serves callers that cannot
+ * on, held until the process ends) instead of pinned blocks that grow with
+ * the calls.  No counterpart in the reference: it serves callers that cannot
  * allocate device memory (code under HIP graph capture, serving loops,
  * harnesses that forbid hipMalloc).  Rejects n_gp > SMA160_NOALLOC_MAX_GP
  * and n_mat > SMA160_NOALLOC_MAX_MAT with SMA_ERR_ARG.  Calls that overlap
