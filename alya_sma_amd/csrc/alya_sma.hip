@@ -52,7 +52,11 @@ unsigned nblocks(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 
 // Steps per captured graph of a long run, longest first (even lengths: see
 // sld_dev_step); each run pays one stand-alone predictor.
-constexpr int GRAPH_RUNS[] = {64, 16, 2};
+// Lengths of captured runs, taken greedily: any number of steps is 64s, at most
+// three 16s, then at most one 8, 4, 2 and one eager step.  A launch of a run costs ~10 us
+// beyond its kernels (8 steps of a small mesh: 103 us as one run, 128 as four
+// of 2); longer runs than 64 gain nothing.
+constexpr int GRAPH_RUNS[] = {64, 16, 8, 4, 2};
 
 struct GraphKey {
   double dt, phi;
@@ -1454,7 +1458,7 @@ int sld_dev_prepare(sld_dev* d, double dt, int32_t scheme, double phi, int64_t n
 int sld_dev_step(sld_dev* d, double dt, int32_t scheme, double phi, int64_t nsteps) {
   if (int rc = step_checks(d, scheme, dt, nsteps)) return rc;
   int64_t left = nsteps;
-  // runs of 64, 16 and 2 steps replay captured graphs (an even length
+  // runs of 64, 16, 8, 4 and 2 steps replay captured graphs (an even length
   // returns the history and clock slots to where they started); inside a run
   // each corrector also predicts the next step
   for (int len : GRAPH_RUNS) {
