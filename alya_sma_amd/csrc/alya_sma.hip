@@ -78,7 +78,9 @@ struct sld_dev {
   std::vector<int32_t> color_ptr;   // [ncolor+1] ranges of color_list
   std::vector<int32_t> color_list;  // stored elements sorted by colour (stable)
   std::vector<int32_t> order;       // stored position -> caller element
-  int32_t* stored_dev = nullptr;    // caller element -> stored position (null: the same), for read-back
+  int32_t* stored_dev = nullptr;    // caller element -> stored position (null: the same), for read-back;
+                                    // made at creation, on the handle's device, so that reading a field
+                                    // changes nothing of the handle, whatever thread reads it
   int32_t* color_list_dev = nullptr;
   // device arrays
   int32_t* lnods = nullptr;
@@ -706,18 +708,6 @@ struct DeviceScope {
   }
 };
 
-// Uploads the stored position of each element when it differs (once).
-int stored_positions(sld_dev* d) {
-  if (d->stored_dev || d->nh_begin < 0) return 0;
-  std::vector<int32_t> pos((size_t)d->nelem);
-  for (int64_t i = 0; i < d->nelem; ++i) pos[d->order[i]] = (int32_t)i;
-  int32_t* p = nullptr;
-  if (int rc = upload(&p, pos.data(), pos.size(), d->stream)) return rc;
-  track(d, p);
-  d->stored_dev = p;
-  return 0;
-}
-
 // Rows of a result from the device to the caller's array: `launch` packs rows
 // row0 .. row0 + m - 1 into a slot of the stage, the host copies them out.
 // Before, each component was copied to a host vector and the components
@@ -1104,6 +1094,9 @@ int sld_dev_create(const sld_mesh_desc* mesh, const sld_material_desc* mat,
     TRY(upload(&d->law_of_elem, le.data(), le.size(), s)); track(d, d->law_of_elem);
     // stored grouped by law: the neo-Hookean elements are a trailing range
     d->nh_begin = (int32_t)(std::find(le.begin(), le.end(), (uint8_t)1) - le.begin());
+    std::vector<int32_t> pos((size_t)ne);
+    for (int64_t i = 0; i < ne; ++i) pos[d->order[i]] = (int32_t)i;
+    TRY(upload(&d->stored_dev, pos.data(), pos.size(), s)); track(d, d->stored_dev);
   }
   hipLaunchKernelGGL(sld::sld_elem_moduli, dim3(nblocks(ne, 256)), dim3(256), 0, s, ne, d->props,
                      d->mat_of_elem, d->E_of_elem, d->kg);
@@ -1707,7 +1700,6 @@ int sld_dev_get(sld_dev* d, int32_t field, void* host, int64_t count) {
       const void* src[3] = {d->sdv[k_slot][0], d->sdv[k_slot][1], d->sdv[k_slot][2]};
       // F_SA of the SMA elements (stored first) is F_AS
       const int64_t same = !d->one_f ? 0 : 8 * (int64_t)(d->nh_begin >= 0 ? d->nh_begin : ne);
-      if (int rc = stored_positions(d)) return rc;
       return get_rows<3>(d, src, false, d->stored_dev, ngp, host, same);
     }
     case SLD_FIELD_REACTIONS: {
@@ -1756,7 +1748,6 @@ int sld_dev_get(sld_dev* d, int32_t field, void* host, int64_t count) {
       const double* f = field == SLD_FIELD_PK1 ? d->P_out : d->S_out;
       const void* src[9];
       for (int k = 0; k < 9; ++k) src[k] = f + k * ngp;
-      if (int rc = stored_positions(d)) return rc;
       return get_rows<9>(d, src, false, d->stored_dev, ngp, host);
     }
     case SLD_FIELD_FLAGS: {
