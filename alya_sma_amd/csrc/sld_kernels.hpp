@@ -1540,7 +1540,7 @@ __global__ void __launch_bounds__(EPB * 8, (ElemOccupancy<R, LAWS, DAMP, STORE>:
 
     if constexpr (STORE) {
       R Fi[9], S[9];
-      sma::inv3<R>(Fm, Fi);
+      sma::inv3<R, true>(Fm, Fi);
       sma::pk2<R>(Fi, tau, S);
       const int64_t ngp = A.nelem * 8, gp = (int64_t)e * 8 + lb;
       if (valid) {
@@ -1820,7 +1820,7 @@ __global__ void __launch_bounds__(256) sma160_points(LawArgs A) {
   if constexpr (!FP32_KIN) {
     double tau[6], Fi[9];
     rm = sma::law_point(m, F, xS0, FAS0, FSA0, tau);
-    double det = sma::inv3<double>(F, Fi);
+    double det = sma::inv3<double, true>(F, Fi);
     if (!(det > 0.0)) rm.flags |= sma::FLAG_DETF_NONPOS;
     sma::pk2<double>(Fi, tau, S);
   } else {

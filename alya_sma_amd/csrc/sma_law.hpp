@@ -118,8 +118,9 @@ __host__ __device__ __forceinline__ float fast_rcp(float x) {
 
 // 1/x in FP64 for the element step: the hardware estimate refined by two
 // Newton steps, within 1 ulp (the IEEE division: 0.5) in 5 instructions
-// against its 11.  Zero and non-finite x give NaN or infinity; a state that
-// holds one stops the run in any case.
+// against its 11.  0, infinities and an x whose reciprocal overflows give NaN
+// (0 times infinity in the steps), which the step's health check treats as it
+// does infinity.  Not for values that a caller is handed (inv3's EXACT).
 __host__ __device__ __forceinline__ double rcp64(double x) {
 #if defined(__HIP_DEVICE_COMPILE__)
   double y = __builtin_amdgcn_rcp(x);
@@ -1146,13 +1147,17 @@ __host__ __device__ __forceinline__ R det3(const R (&M)[9]) {
          M[6] * (M[1] * M[5] - M[2] * M[4]);
 }
 
-// Column-major 3x3 inverse by cofactors (one reciprocal, 1 ulp); returns det.
-template <typename R>
+// Column-major 3x3 inverse by cofactors (one reciprocal); returns det.  EXACT:
+// the IEEE reciprocal in FP64, so that a singular M gives the infinities of a
+// division by 0; else 1 ulp, for values of the element step.
+template <typename R, bool EXACT = false>
 __host__ __device__ __forceinline__ R inv3(const R (&M)[9], R (&Mi)[9]) {
   R C[9];
   cof3<R>(M, C);
   const R det = M[0] * C[0] + M[3] * C[3] + M[6] * C[6];
-  const R r = rcp_r<R>(det);
+  R r;
+  if constexpr (EXACT && sizeof(R) == 8) r = R(1) / det;
+  else r = rcp_r<R>(det);
 #pragma unroll
   for (int i = 0; i < 3; ++i)
 #pragma unroll
