@@ -1960,21 +1960,29 @@ int sma160_eval(int64_t n, int32_t n_mat, const double* props, const int32_t* ma
   HostLease lease;
   if (int rc = lease.take()) return rc;
   HostStage& st = *lease.st;
-  // equal chunks of whole waves; a slot holds a chunk's sections, inputs first.
+  // Equal chunks of whole waves; a slot holds a chunk's sections, inputs first.
   // A chunk's outputs are stored before a later chunk's inputs are read: fine
-  // for distinct arrays and for a call in place, one chunk for other overlaps.
-  auto meet = [&](const void* out, size_t bo, const void* in, size_t bi) {
-    const char *x = (const char*)out, *y = (const char*)in;
-    return in && x != y && x < y + bi && y < x + bo;
-  };
+  // for distinct arrays and where the history or the stresses take the place of
+  // their own inputs (a chunk then overwrites what it has read).  Any other
+  // overlap takes one chunk: everything is read, then the history, the stresses
+  // and the flags are stored, whole and in this order.
   const size_t rows = (size_t)n * 8;
-  auto meets_inputs = [&](const void* out, size_t bo) {
-    return out && (meet(out, bo, F, 9 * rows) || meet(out, bo, sdv_old, 3 * rows) ||
-                   meet(out, bo, E_of_gp, rows) || meet(out, bo, mat_of_gp, rows / 2) ||
-                   out == (const void*)E_of_gp || out == (const void*)mat_of_gp);
+  struct Range {
+    const void* at;
+    size_t bytes;
   };
-  const bool whole = meets_inputs(sdv_new, 3 * rows) || meets_inputs(S, 9 * rows) ||
-                     meets_inputs(flags, rows / 2) || (const void*)sdv_new == F || (const void*)S == sdv_old;
+  auto meet = [](Range x, Range y) {
+    const char *p = (const char*)x.at, *q = (const char*)y.at;
+    return p && q && p < q + y.bytes && q < p + x.bytes;
+  };
+  const Range outs[3] = {{sdv_new, 3 * rows}, {S, 9 * rows}, {flags, rows / 2}};
+  const Range ins[4] = {{sdv_old, 3 * rows}, {F, 9 * rows}, {E_of_gp, rows}, {mat_of_gp, rows / 2}};
+  bool whole = false;
+  for (int k = 0; k < 3; ++k) {
+    for (int j = 0; j < 4; ++j)
+      if (!(k == j && k < 2 && outs[k].at == ins[j].at)) whole = whole || meet(outs[k], ins[j]);
+    for (int j = 0; j < k; ++j) whole = whole || meet(outs[k], outs[j]);
+  }
   int64_t nchunk = whole ? 1 : (n + kEvalChunk - 1) / kEvalChunk;
   const int64_t per = nchunk == 1 ? n : ((n + nchunk - 1) / nchunk + 63) / 64 * 64;
   nchunk = (n + per - 1) / per;
