@@ -13,11 +13,27 @@
 
 #include "alya_sma.h"
 #include "common.hpp"
+#include "once_per_device.hpp"
 #include "surrogate.hpp"
 
 namespace {
 #define SCHK(x) SMA_HIPCHK(x)
 unsigned nb(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs); }
+
+// The dynamic LDS limit of `kernel` on the current device (a limit holds for
+// one device), whose CU count is returned.
+int lds_limit(sma_abi::OncePerDevice& once, const void* kernel, int bytes, int* ncu = nullptr) {
+  int dev = 0;
+  SCHK(hipGetDevice(&dev));
+  if (ncu) (void)hipDeviceGetAttribute(ncu, hipDeviceAttributeMultiprocessorCount, dev);
+  return once(dev, [&]() -> int {
+    SCHK(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
+    return SMA_OK;
+  });
+}
+sma_abi::OncePerDevice g_infer_lds, g_train_lds;
+
+int infer_lds(int* ncu) { return lds_limit(g_infer_lds, (const void*)mlp::mlp_infer, (int)mlp::INF_SMEM, ncu); }
 }  // namespace
 
 struct sma_mlp {
@@ -62,12 +78,7 @@ mlp::AdamArgs adam_args(sma_mlp* m, int parts) {
 int train_pass(sma_mlp* m, int64_t n, const float* X, const float* T, int* parts_out, hipStream_t s) {
   if (n > (int64_t)INT32_MAX * mlp::TR_ROWS)
     return sma_abi::fail(SMA_ERR_ARG, "sma_mlp: mini-batch too large");
-  static bool attr = false;
-  if (!attr) {
-    SCHK(hipFuncSetAttribute((const void*)mlp::mlp_train, hipFuncAttributeMaxDynamicSharedMemorySize,
-                             (int)sizeof(mlp::TrainLds)));
-    attr = true;
-  }
+  if (int rc = lds_limit(g_train_lds, (const void*)mlp::mlp_train, (int)sizeof(mlp::TrainLds))) return rc;
   const int64_t chunks = (n + mlp::TR_ROWS - 1) / mlp::TR_ROWS;
   const int parts = (int)std::min<int64_t>(chunks, mlp::TR_MAX_GRID);
   if (int rc = grow(m, parts)) return rc;
@@ -177,16 +188,9 @@ int sma_mlp_forward_device(sma_mlp* m, int64_t n, const float* X, float* Y, void
   if (!m || n < 0 || (n > 0 && (!X || !Y))) return sma_abi::fail(SMA_ERR_ARG, "sma_mlp_forward_device: bad arguments");
   if (n > INT32_MAX) return sma_abi::fail(SMA_ERR_ARG, "sma_mlp_forward_device: n must be below 2^31");
   if (n == 0) return SMA_OK;
-  static bool attr = false;
-  if (!attr) {
-    SCHK(hipFuncSetAttribute((const void*)mlp::mlp_infer, hipFuncAttributeMaxDynamicSharedMemorySize,
-                             (int)mlp::INF_SMEM));
-    attr = true;
-  }
+  int ncu = 256;
+  if (int rc = infer_lds(&ncu)) return rc;
   const int64_t nblk = (n + 15) / 16;   // the smallest row blocks
-  int dev = 0, ncu = 256;
-  (void)hipGetDevice(&dev);
-  (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
   const unsigned grid = (unsigned)std::min<int64_t>(nblk, ncu);
   hipLaunchKernelGGL(mlp::mlp_infer, dim3(grid), dim3(mlp::INF_THREADS), mlp::INF_SMEM, (hipStream_t)stream, m->Wi,
                      m->bp, X, n, (const unsigned*)nullptr, (int64_t)0, Y);
@@ -253,15 +257,8 @@ int sma_mlp_gen_samples_device(int64_t n, uint64_t seed, const double* props_dev
 // are read on the device; seg_cap slots per segment).
 int sma_mlp_infer_listed(sma_mlp* m, const float* X, const unsigned* seg_count, int64_t seg_cap,
                          float* Y, hipStream_t s) {
-  static bool attr = false;
-  if (!attr) {
-    SCHK(hipFuncSetAttribute((const void*)mlp::mlp_infer, hipFuncAttributeMaxDynamicSharedMemorySize,
-                             (int)mlp::INF_SMEM));
-    attr = true;
-  }
-  int dev = 0, ncu = 256;
-  (void)hipGetDevice(&dev);
-  (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
+  int ncu = 256;
+  if (int rc = infer_lds(&ncu)) return rc;
   const int64_t cap = seg_cap * mlp::LIST_SEGS;
   const unsigned grid =
       (unsigned)std::max<int64_t>(1, std::min<int64_t>((cap + 15) / 16, ncu));
