@@ -17,6 +17,7 @@
 
 #include "alya_sma.h"
 #include "common.hpp"
+#include "stage_pool.hpp"
 #include "sld_kernels.hpp"
 
 namespace {
@@ -603,15 +604,17 @@ int enqueue_step(sld_dev* d, double dt, int scheme, double phi, int tn, KernelTi
 // over the host link, so that operands and results need no copy of their own.
 // A transfer goes through kStageSlots slots in turn on two streams: the host
 // fills and empties slots while kernels read and write others.  A call takes a
-// stage from the pool (or makes one) and gives it back; the pool keeps kStagePool
-// of them with blocks up to kStageKeep, which are left to the process's end
-// (freeing after the runtime has shut down is not safe).
-constexpr int kStageSlots = 4, kStagePool = 4;
-constexpr size_t kStageKeep = (size_t)32 << 20;
+// stage from the pool (or makes one) and gives it back.  Making one costs more
+// than a small call, so the pool keeps as many as callers were seen at once, up
+// to kStagePool for a device, with up to kStageKeep bytes of blocks in all, left
+// to the process's end (freeing after the runtime has shut down is not safe).
+constexpr int kStageSlots = 4;
+constexpr size_t kStagePool = 64, kStageKeep = (size_t)256 << 20;
 struct HostStage {
   int device = -1;
   char* host = nullptr;             // pinned; the device uses the same address
   size_t bytes = 0;
+  HostStage* next = nullptr;        // in the pool
   hipStream_t stream[2] = {nullptr, nullptr};
   hipEvent_t done[kStageSlots] = {nullptr, nullptr, nullptr, nullptr};
 
@@ -619,9 +622,7 @@ struct HostStage {
     if (want <= bytes) return SMA_OK;
     size_t nb = bytes ? bytes : 4096;
     while (nb < want) nb *= 2;
-    if (host) (void)hipHostFree(host);
-    host = nullptr;
-    bytes = 0;
+    drop_block();
     void* p = nullptr;
     HIPCHK(hipHostMalloc(&p, nb, hipHostMallocMapped | hipHostMallocCoherent));
     host = (char*)p;
@@ -629,6 +630,11 @@ struct HostStage {
     if (p != host) return fail(SMA_ERR_HIP, "host stage: pinned memory has no common address");
     bytes = nb;
     return SMA_OK;
+  }
+  void drop_block() {
+    if (host) (void)hipHostFree(host);
+    host = nullptr;
+    bytes = 0;
   }
   int open(int dev) {
     device = dev;
@@ -641,11 +647,10 @@ struct HostStage {
       if (e) (void)hipEventDestroy(e);
     for (auto& q : stream)
       if (q) (void)hipStreamDestroy(q);
-    if (host) (void)hipHostFree(host);
+    drop_block();
   }
 };
-std::mutex g_stage_mu;
-HostStage* g_stage_pool[kStagePool] = {};
+sma_abi::StagePool<HostStage> g_stages(kStagePool, kStageKeep);
 
 // A stage of the current device, given back (its streams idle) when the
 // call ends.
@@ -656,15 +661,7 @@ class HostLease {
   int take() {
     int dev = 0;
     HIPCHK(hipGetDevice(&dev));
-    {
-      std::lock_guard<std::mutex> lock(g_stage_mu);
-      for (auto& p : g_stage_pool)
-        if (p && p->device == dev) {
-          st = p;
-          p = nullptr;
-          return SMA_OK;
-        }
-    }
+    if ((st = g_stages.take(dev))) return SMA_OK;
     st = new (std::nothrow) HostStage();
     if (!st) return fail(SMA_ERR_HIP, "host stage: out of memory");
     return st->open(dev);
@@ -673,19 +670,8 @@ class HostLease {
     if (!st) return;
     if (busy)
       for (auto& q : st->stream) (void)hipStreamSynchronize(q);
-    if (st->bytes > kStageKeep) {
-      (void)hipHostFree(st->host);
-      st->host = nullptr;
-      st->bytes = 0;
-    }
-    {
-      std::lock_guard<std::mutex> lock(g_stage_mu);
-      for (auto& p : g_stage_pool)
-        if (!p && st->done[kStageSlots - 1]) {
-          p = st;
-          return;
-        }
-    }
+    // a stage whose making failed is not kept
+    if (st->done[kStageSlots - 1] && g_stages.give(st)) return;
     st->close();
     delete st;
   }
@@ -1917,7 +1903,8 @@ int sld_dev_destroy(sld_dev* d) {
 // points, in chunks, 225 us a call against 455 (chunks of 4096 and 16384: 288
 // and 295).  The material rows are read from there too (250 us with the 64 rows
 // copied to the device first).
-// Memory: at most 212 bytes x kEvalChunk x kStageSlots (5 MB) and the material rows.
+// Memory: the power of two above 212 bytes x kEvalChunk x kStageSlots (5.2 MB) and
+// the material rows; a call whose arrays overlap takes 212 bytes a point at once.
 constexpr int64_t kEvalChunk = 6144;
 
 static int law_launch(int64_t n, int32_t nmat, const double* props, const int32_t* mat, const double* E,

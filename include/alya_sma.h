@@ -53,9 +53,13 @@ const char *sma_last_error(void);
  *   out; S [9][n_gp] second Piola-Kirchhoff out; flags [n_gp] out (may be NULL).
  * precision: 0 = FP64, 1 = FP32 spectral/stress with FP64 return map.
  * Host pointers; synchronous.  The kernel reads and writes pinned host memory
- * that a call takes from a small pool (at most 4 blocks of up to 32 MB, held to
- * the process's end), so that repeated calls allocate nothing.  Outputs may
- * take the place of inputs (sdv_new = sdv_old, S = F).
+ * that a call takes from a pool.  The pool grows with the calls that run at once
+ * and is held to the process's end: up to 64 blocks for each device, 256 MB in
+ * all, so that repeated calls within these bounds allocate nothing.  A block is
+ * the power of two above 5.2 MB and the material rows, less for small calls.
+ * Outputs may take the place of inputs (sdv_new = sdv_old, S = F); arrays that
+ * overlap otherwise are staged whole (212 bytes a point): all inputs are read
+ * before sdv_new, S and flags are stored, in this order.
  * ------------------------------------------------------------------------ */
 int sma160_eval(int64_t n_gp, int32_t n_mat, const double *props,
                 const int32_t *mat_of_gp, const double *E_of_gp,
