@@ -1096,12 +1096,19 @@ __host__ __device__ __forceinline__ void kirchhoff(const Mat& m, const Spectral<
 // spectral form's are relative to 1.  The spectral form, which follows the
 // reference operation by operation, stays where the series does not reach
 // (stretches beyond about 1/2..2, non-finite or singular F), for deviatoric
-// strains up to 1e-5 (there its own rounding, 1e-16, is seen in the direction
-// e'/|e'| and so in the stress of a transformed point), where the return map
-// needs the reference's iteration, whose count and end can hang on the last
-// bit, and where an off-diagonal of b is so small (1e-162 .. 1e-77 beside any
-// stretch) that the reference's Householder step underflows: its NaN is kept.
+// strains up to 1e-5 of a point with a history (there its own rounding, 1e-16, is
+// seen in the direction e'/|e'| and so in the stress), for a rotation's strains of
+// rounding size, where the return map needs the reference's iteration, whose count
+// and end can hang on the last bit, and where an off-diagonal of b is so small
+// (1e-162 .. 1e-77 beside any stretch) that the reference's Householder step
+// underflows: its NaN is kept.
+// Points at rest (xS = 0, loading function well below its threshold), as much of a
+// loaded body is, take the series also below 1e-5 and at F = I: no direction enters
+// their stress.  A wave that holds points of both kinds goes through both forms:
+// 500 points, 2% of them at rest, 14.4 us with the spectral form for those, 4.2 with
+// the series for all, 8.3 with the spectral form for all.
 constexpr double kSeriesMinEn = 1.0e-5, kSeriesMinB = 1.0e-60;
+constexpr double kNoiseEn = 1.0e-13, kNoiseTurn = 1.0e-10;
 __host__ __device__ __forceinline__ ReturnMap law_point(const Mat& m, const double (&F)[9], double xS_0,
                                                         double F_AS_0, double F_SA_0, double (&tau)[6]) {
   ReturnMap rm;
@@ -1113,8 +1120,15 @@ __host__ __device__ __forceinline__ ReturnMap law_point(const Mat& m, const doub
     const bool under = tiny(F[0] * F[1] + F[3] * F[4] + F[6] * F[7]) ||
                        tiny(F[0] * F[2] + F[3] * F[5] + F[6] * F[8]) ||
                        tiny(F[1] * F[2] + F[4] * F[5] + F[7] * F[8]);
-    if (h.ok && h.e_n > kSeriesMinEn && !under) {
+    if (h.ok && !under) {
       done = return_map_closed(m, h.theta, h.e_n, xS_0, F_AS_0, F_SA_0, rm);
+      // small strains: at rest (F_AS is that of the strain) by a margin that no
+      // rounding of either form crosses, and not a rotation alone (a half turn's b is
+      // exact in both forms)
+      const double turn = fmax(fmax(fabs(H[1]), fabs(H[2])), fabs(H[5]));
+      const bool rest = xS_0 == 0.0 && rm.flags == 0 && m.Rs_AS - rm.F_AS > 1.0e-9 * m.G &&
+                        (h.e_n > kNoiseEn || turn <= kNoiseTurn);
+      done = done && (h.e_n > kSeriesMinEn || rest);
       kirchhoff_hencky64(m, h, rm.xS, tau);
     }
   }

@@ -1,0 +1,90 @@
+"""Points at rest (no martensite, loading function below its threshold) of the
+point-wise FP64 law, compiled for the host from the device header, at strains from
+1e-16 to 1e-5: their stresses are as exact as the strain is, the series' relative
+accuracy instead of the spectral form's absolute 1e-16 (and a seventh of its
+operations).
+
+Bound: b - I is formed from H = F - I by sums of at most eight rounded terms of size
+|H|, the series' reciprocal and polynomial add ~20 more roundings relative to |E|, the
+stress and its pull-back (F within 1e-5 of I) as many again: 64 eps |H| (2G + 3K)
+covers them.  The exact strain is E = Z + Z^3/3 + ..., Z = (b - I)(b + I)^-1 in
+extended precision."""
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+HIPCC = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "bin", "hipcc")
+SRC = r'''
+#include "sma_law.hpp"
+#include <cstdio>
+using namespace sma;
+int main() {
+  double b[27];
+  while (fread(b, 8, 27, stdin) == 27) {
+    double F[9], Fi[9], tau[6], o[10];
+    for (int i = 0; i < 9; ++i) F[i] = b[18 + i];
+    const ReturnMap r = law_point(make_mat(b, b[0]), F, 0.0, 0.0, 0.0, tau);
+    inv3<double, true>(F, Fi);
+    pk2<double>(Fi, tau, (double(&)[9])o[0]);
+    o[9] = r.flags;
+    fwrite(o, 8, 10, stdout);
+  }
+  return 0;
+}
+'''
+NITINOL = np.array([60000, 0.33, 0.05, 400, 500, 0, 0, 0, 0, 250, 150, 0, 0, 0, 0, 1, 1, 0.0])
+
+
+@pytest.fixture(scope="module")
+def prog(tmp_path_factory):
+    if not os.path.exists(HIPCC):
+        pytest.skip("hipcc not available")
+    d = tmp_path_factory.mktemp("rest")
+    (d / "r.cpp").write_text(SRC)
+    subprocess.run([HIPCC, "-x", "hip", "--offload-host-only", "-O2", "-std=c++17",
+                    "-I" + os.path.join(ROOT, "alya_sma_amd", "csrc"), str(d / "r.cpp"), "-o",
+                    str(d / "r")], check=True, capture_output=True)
+
+    def run(P, F):
+        b = np.concatenate([P, F.transpose(0, 2, 1).reshape(-1, 9)], 1)
+        o = subprocess.run([str(d / "r")], input=np.ascontiguousarray(b).tobytes(), capture_output=True, check=True)
+        o = np.frombuffer(o.stdout).reshape(-1, 10)
+        return o[:, :9].reshape(-1, 3, 3), o[:, 9]
+    return run
+
+
+def _inverse(m):
+    c = np.cross(m[:, [1, 2, 0]], m[:, [2, 0, 1]])      # rows of cofactors
+    return c.transpose(0, 2, 1) / (m[:, 0] * c[:, 0]).sum(1)[:, None, None]
+
+
+@pytest.mark.parametrize("unit", [1.0, 1e6])
+@pytest.mark.parametrize("size", [1e-16, 1e-12, 1e-9, 1e-7, 2e-6])
+def test_stress_of_a_point_at_rest(prog, size, unit):
+    n = 2000
+    r = np.random.default_rng(1)
+    P = np.tile(NITINOL, (n, 1))
+    P[:, [0, 3, 4, 9, 10]] *= r.uniform(0.9, 1.1, (n, 5)) * unit
+    F = np.eye(3) + size * r.normal(size=(n, 3, 3))
+    S, fl = prog(P, F)
+    F = F.astype(np.longdouble)
+    H = F - np.eye(3)
+    c = H + H.transpose(0, 2, 1) + H @ H.transpose(0, 2, 1)
+    Z = c @ _inverse(c + 2 * np.eye(3))
+    E = Z + Z @ Z @ Z / 3
+    th = np.trace(E, axis1=1, axis2=2)[:, None, None] * np.eye(3)
+    nu, G2, K = P[:, 1], P[:, 0] / (1 + P[:, 1]), P[:, 0] / (3 * (1 - 2 * P[:, 1]))
+    tau = K[:, None, None] * th + G2[:, None, None] * (E - th / 3)
+    Fi = _inverse(F)
+    exact = Fi @ tau @ Fi.transpose(0, 2, 1)
+    tol = 64 * 2.0 ** -52 * np.abs(H).max((1, 2)) * (G2 + 3 * K)
+    assert (fl == 0).all() and (nu < 0.5).all()
+    assert (np.abs(S - exact).max((1, 2)) <= tol).all()
+
+
+def test_undeformed_point_has_no_stress(prog):
+    S, fl = prog(NITINOL[None], np.eye(3)[None])
+    assert (S == 0.0).all() and (fl == 0).all()
