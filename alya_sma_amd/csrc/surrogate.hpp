@@ -95,10 +95,11 @@ __device__ __forceinline__ float silu(float z) {
 // s = sigmoid(z) to half an ulp or so (one Newton step on the hardware
 // reciprocal), silu(z) = z s and silu'(z) = s (1 + z (1 - s)).
 __device__ __forceinline__ void silu_both(float z, float& y, float& g) {
-  const float t = 1.0f + __expf(fminf(-z, 85.0f));   // finite: silu(-85) ~ 1e-35
+  const float t = 1.0f + __expf(-z);
   float s = __builtin_amdgcn_rcpf(t);
   y = z * s;
-  s = fmaf(fmaf(-t, s, 1.0f), s, s);
+  // t is infinite below z = -88: s and both results are then 0, however large -z
+  s = fmaf(fmaf(-fminf(t, 0x1.fffffep127f), s, 1.0f), s, s);
   g = s * (1.0f + z * (1.0f - s));
 }
 
