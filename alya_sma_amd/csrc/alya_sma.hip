@@ -1810,20 +1810,29 @@ int sld_dev_set(sld_dev* d, int32_t field, const void* host, int64_t count) {
     case SLD_FIELD_SDV: {
       if (count != 3 * ngp) return fail(SMA_ERR_ARG, "count does not match field size");
       const double* in = (const double*)host;
-      tmp.resize(ngp);
+      // the components parted in one pass over the caller's array, which also says
+      // whether the SMA elements' (stored first) two loading functions are one
+      tmp.resize(3 * ngp);
+      double *x = tmp.data(), *f1 = x + ngp, *f2 = f1 + ngp;
       const int64_t nsma = d->nh_begin >= 0 ? d->nh_begin : ne;
-      d->one_f = d->finite_c;
-      for (int64_t i = 0; i < nsma && d->one_f; ++i)
+      uint64_t differ = 0;
+      for (int64_t i = 0; i < ne; ++i) {
+        const double* q = in + 24 * (int64_t)d->order[i];
+        uint64_t a[8], b[8], c = 0;
         for (int g = 0; g < 8; ++g) {
-          const double* f = in + (8 * (int64_t)d->order[i] + g) * 3;
-          d->one_f = d->one_f && std::memcmp(f + 1, f + 2, sizeof(double)) == 0;
+          x[8 * i + g] = q[3 * g];
+          f1[8 * i + g] = q[3 * g + 1];
+          f2[8 * i + g] = q[3 * g + 2];
         }
-      for (int k = 0; k < 3; ++k) {
-        for (int64_t i = 0; i < ne; ++i)
-          for (int g = 0; g < 8; ++g) tmp[8 * i + g] = in[(8 * (int64_t)d->order[i] + g) * 3 + k];
-        for (int sl = 0; sl < 2; ++sl)
-          HIPCHK(hipMemcpy(d->sdv[sl][k], tmp.data(), ngp * sizeof(double), hipMemcpyHostToDevice));
+        std::memcpy(a, f1 + 8 * i, sizeof(a));
+        std::memcpy(b, f2 + 8 * i, sizeof(b));
+        for (int g = 0; g < 8; ++g) c |= a[g] ^ b[g];
+        if (i < nsma) differ |= c;
       }
+      d->one_f = d->finite_c && differ == 0;
+      for (int k = 0; k < 3; ++k)
+        for (int sl = 0; sl < 2; ++sl)
+          HIPCHK(hipMemcpy(d->sdv[sl][k], x + k * ngp, ngp * sizeof(double), hipMemcpyHostToDevice));
       return SMA_OK;
     }
     case SLD_FIELD_TIME:
