@@ -52,11 +52,11 @@ unsigned nblocks(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 }  // namespace
 
 // Steps per captured graph of a long run, longest first (even lengths: see
-// sld_dev_step); each run pays one stand-alone predictor.
-// Lengths of captured runs, taken greedily: any number of steps is 64s, at most
-// three 16s, then at most one 8, 4, 2 and one eager step.  A launch of a run costs ~10 us
-// beyond its kernels (8 steps of a small mesh: 103 us as one run, 128 as four
-// of 2); longer runs than 64 gain nothing.
+// sld_dev_step); each run pays one stand-alone predictor.  Taken greedily: any
+// number of steps is 64s, at most three 16s, then at most one 8, 4, 2 and one
+// eager step.  A launch of a run costs ~10 us beyond its kernels (8 steps of a
+// small mesh: 103 us as one run, 128 as four of 2); longer runs than 64 gain
+// nothing.
 constexpr int GRAPH_RUNS[] = {64, 16, 8, 4, 2};
 
 struct GraphKey {
@@ -1908,10 +1908,13 @@ int sld_dev_destroy(sld_dev* d) {
 // sma160_eval's points go through a stage: the law reads every input once and
 // writes every output once, in runs of 512 bytes a wave, so nothing is gained by
 // having them in device memory first.  8 points take 12 us against 32 for an
-// upload, a launch and a download (a call from Python 20 against 39); 40001
-// points, in chunks, 225 us a call against 455 (chunks of 4096 and 16384: 288
-// and 295).  The material rows are read from there too (250 us with the 64 rows
-// copied to the device first).
+// upload, a launch and a download (a call from Python 20 against 39).  The material
+// rows are read from there too (64 rows copied to the device first cost 20 us more
+// than they save; a row for each of 40001 points still takes 471 us a call, 612 with
+// an upload).  Calls of 40001 points 455 -> 230 us.  Chunks of 6144 points are within
+// 8% of the best length from 7000 to 60000 points (us a call in chunks of 4096, 6144,
+// 8192 and 16384: 12288 points 96, 100, 101, 115; 20000 131, 127, 135, 146; 60000
+// 408, 377, 371, 351); a call of millions would gain 10 to 30% from longer ones.
 // Memory: the power of two above 212 bytes x kEvalChunk x kStageSlots (5.2 MB) and
 // the material rows; a call whose arrays overlap takes 212 bytes a point at once.
 constexpr int64_t kEvalChunk = 6144;
@@ -2129,7 +2132,7 @@ extern "C" int sma160_eval_noalloc(int64_t n, int32_t n_mat, const double* props
   if (mat_of_gp) HIPCHK(hipMemcpy(d_mat, mat_of_gp, (size_t)n * sizeof(int32_t), hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(d_F, F, (size_t)9 * n * sizeof(double), hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(d_sold, sdv_old, (size_t)3 * n * sizeof(double), hipMemcpyHostToDevice));
-  // the null stream, as sma160_eval
+  // the null stream
   if (int rc = law_launch(n, n_mat, d_props, mat_of_gp ? d_mat : nullptr, E_of_gp ? d_E : nullptr,
                           d_F, d_sold, d_snew, d_S, flags ? d_flags : nullptr, precision, nullptr))
     return rc;

@@ -936,13 +936,16 @@ __device__ __forceinline__ void wave_sync() {
 }
 
 // EPB elements per block, 8 threads (one per Gauss point) per element.
-// What bounds it: VALU issue, 87% of the busy cycles in FP64 at ~2.05 GHz (C1:
-// 663 instructions a wave, 3 of 4 in FP64) and 99% in FP32 (675); the rest the
-// first loads of a wave and the launch's start and end.  In FP64 an element's
-// lanes exchange values by DPP moves (hex_grad, hex_grad_t) instead of through LDS: with Walsh-Hadamard
-// sums and Gauss-point rows in LDS (175 FP64 values read or written per lane)
-// the LDS of a CU, shared by its four SIMDs, was as busy as the VALU, and the
-// two overlapped poorly.  FP64 element launch, before -> with exchanges: C1
+// What bounds it (counters): in FP64 on C1, whose state stays in the 256 MB cache,
+// VALU issue, 0.86 of the busy cycles (663 instructions a wave, 3 of 4 in FP64, 4
+// cycles each); on meshes whose state does not (631 000 elements and more) it
+// issues 0.5 to 0.6, as much of a wave's time being waits for memory at 2.7 TB/s.
+// FP32 (675 instructions) issues one in 4 cycles on C1 and 0.9 beyond the cache with
+// 4 waves a SIMD; that is no ceiling (the neo-Hookean launch reaches 1.3 with 8).
+// In FP64 an element's lanes exchange values by DPP moves (hex_grad, hex_grad_t)
+// instead of through LDS: with Walsh-Hadamard sums and Gauss-point rows in LDS
+// (175 FP64 values read or written per lane) the LDS of a CU, shared by its four
+// SIMDs, was as busy as the VALU, and the two overlapped poorly.  FP64 element launch, before -> with exchanges: C1
 // 400x20x20 46.7 -> 39.2 us; 631 000 elements in 64 specimens 191 -> 167;
 // 691 000 elements of SMA tube in tissue 159 -> 125; 2583 damped elements
 // 8.0 -> 6.5.
@@ -1783,7 +1786,10 @@ __global__ void __launch_bounds__(256) sld_pack(PackArgs A) {
 // again, and the inputs of a call, or what its caller just wrote, stay in.
 // 1.28 million points, 256 materials: 125 us with the spectral form at every
 // point, 54 with the series strain, 41 with the streaming stores (the inputs
-// then fit the 256 MB cache; loads past the caches: 59; workgroups of 64: 57).
+// then fit the 256 MB cache; loads past the caches: 59).  Five sets of inputs in
+// turn, plain -> streaming stores: 300 000 points 18.9 -> 12.8 us, 640 000 33.5 ->
+// 32.8, 1.28 million 61.4 -> 60.3; with a kernel after each that reads S back, which
+// it then has to fetch from memory, 26.8 -> 28.4, 47.8 -> 50.7 and 94.5 -> 96.4.
 // ----------------------------------------------------------------------------
 struct LawArgs {
   int64_t n;

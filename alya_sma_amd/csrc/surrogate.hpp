@@ -108,12 +108,13 @@ __device__ __forceinline__ void silu_both(float z, float& y, float& g) {
 // workgroup, one launch per mini-batch.  What bounds it at 16384 rows (256
 // workgroups, one per CU): the chain of ~14 phases between barriers, each a
 // load or LDS read, 8 MFMA deep, an activation and an LDS write (a 1000-row
-// batch, 16 workgroups, takes 25 us; the activations are 4 us of it, the bias
-// sums 1), then writing the partial gradients (213 KB a workgroup, 54 MB, 7
-// us; reduce_adam reads them once).  Neither the 5.2 GFLOP (4 us at the rate of
-// a large BF16 product) nor the 1.8 MB of samples count.  Separate launches
+// batch, 16 workgroups, takes 27 us; the activations are 4 us of it, the bias
+// sums 1; counters: a wave waits 58% of its time, the VALU is busy 0.27 and the
+// matrix cores 0.07), then writing the partial gradients (213 KB a workgroup, 54
+// MB, 7 us; reduce_adam reads them once).  Neither the 5.2 GFLOP (4 us at the rate
+// of a large BF16 product) nor the 1.8 MB of samples count.  Separate launches
 // per layer, product and activation with FP32 intermediates in memory took 930
-// us for those rows (45 launches, 0.5 GB); this takes 34, reduce_adam 14.
+// us for those rows (45 launches, 0.5 GB); this takes 35, reduce_adam 13.
 // Half as many workgroups (and partials) take 1.5 times as long; loading the
 // biases, targets and output weights ahead spills and gains nothing.
 //   Products are formed as in the inference kernel (weights or their transposes
@@ -528,13 +529,15 @@ __global__ void pack_params(const float* __restrict__ W, const float* __restrict
 // barrier), and LDS holds only the weights: 121 KB, one workgroup per CU.
 // A wave carries two 16-row blocks (each A fragment read from LDS feeds two
 // MFMA) in 228 VGPRs, so the workgroup has 8 waves, two per SIMD: one
-// wave's SiLU epilogue (two quarter-rate transcendentals per activation,
-// the kernel's largest cost) overlaps the other's MFMA.  What bounds it: those, 44
-// cycles an activation, 30 us of VALU time for 200 000 rows (their products take
-// 9 of the matrix cores').  Waves take 32-row blocks round robin over the grid
-// (block k on workgroup k mod grid), so a short list spreads over every CU; the
-// rows left after the full rounds go by 16 to a wave when that takes them all,
-// since a wave with a lone 32-row block at the end runs half a round longer.
+// wave's SiLU epilogue (the kernel's largest cost) overlaps the other's MFMA.
+// What bounds it: the VALU is busy 0.60 of the time (counters; 35 cycles an
+// activation, two transcendentals of 8 cycles among them: 23 us for 200 000
+// rows), the matrix cores 0.23 (9 us), and two waves a SIMD leave a part of either
+// and of the LDS reads of the weights uncovered.  Waves take 32-row blocks round
+// robin over the grid (block k on workgroup k mod grid), so a short list spreads
+// over every CU; the rows left after the full rounds go by 16 to a wave when that
+// takes them all, since a wave with a lone 32-row block at the end runs half a
+// round longer.
 // Rows, before -> with 16-row ends: 500 10.4 -> 7.8 us, 16384 11.1 -> 8.7,
 // 200000 44.9 -> 41.5, 400000 80 -> 78; the same where the rest is more than half
 // a round (40000: 15.8).

@@ -74,8 +74,8 @@ int sma160_eval_device(int64_t n_gp, int32_t n_mat, const double *props,
                        double *sdv_new, double *S, uint32_t *flags,
                        int32_t precision, void *stream);
 
-/* Same arguments and results as sma160_eval (host pointers, synchronous,
- * null stream), with no device allocation: the arrays are staged through a
+/* Same arguments and results as sma160_eval (host pointers, synchronous), on
+ * the null stream and with no allocation: the arrays are staged through a
  * fixed array in the library's device memory (3.4 MB on each GPU it runs
  * on, held until the process ends) instead of pinned blocks that grow with
  * the calls.  No counterpart in the reference: it serves callers that cannot
