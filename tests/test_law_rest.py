@@ -88,3 +88,82 @@ def test_stress_of_a_point_at_rest(prog, size, unit):
 def test_undeformed_point_has_no_stress(prog):
     S, fl = prog(NITINOL[None], np.eye(3)[None])
     assert (S == 0.0).all() and (fl == 0).all()
+
+
+SRC_BOTH = r'''
+#include "sma_law.hpp"
+#include <cstdio>
+using namespace sma;
+int main() {
+  double b[30];
+  while (fread(b, 8, 30, stdin) == 30) {
+    double F[9], tau[6], o[20];
+    for (int i = 0; i < 9; ++i) F[i] = b[18 + i];
+    const Mat m = make_mat(b, b[0]);
+    for (int k = 0; k < 2; ++k) {
+      ReturnMap r;
+      if (k == 0) {
+        r = law_point(m, F, b[27], b[28], b[29], tau);
+      } else {
+        const Spectral<double> sp = spectral_fp64(F);
+        r = return_map(m, sp.theta, sp.e_n, b[27], b[28], b[29]);
+        if (!sp.eig_ok) r.flags |= FLAG_EIGEN_FAIL;
+        kirchhoff<double>(m, sp, r.xS, tau);
+      }
+      o[10 * k] = r.xS, o[10 * k + 1] = r.F_AS, o[10 * k + 2] = r.F_SA, o[10 * k + 3] = r.flags;
+      for (int i = 0; i < 6; ++i) o[10 * k + 4 + i] = tau[i];
+    }
+    fwrite(o, 8, 20, stdout);
+  }
+  return 0;
+}
+'''
+
+
+def test_rest_ends_where_the_spectral_form_does(tmp_path):
+    """Thresholds around and far from the strain's loading function (zero and
+    negative ones too), nearly incompressible and auxetic materials, no
+    transformation strain, histories of every kind: the same branch and, at points
+    without an active one or martensite, the same xS and stresses that differ by the spectral form's absolute rounding (64 eps (2G + 3K
+    + 9 |alfa| K))."""
+    if not os.path.exists(HIPCC):
+        pytest.skip("hipcc not available")
+    (tmp_path / "b.cpp").write_text(SRC_BOTH)
+    subprocess.run([HIPCC, "-x", "hip", "--offload-host-only", "-O2", "-std=c++17",
+                    "-I" + os.path.join(ROOT, "alya_sma_amd", "csrc"), str(tmp_path / "b.cpp"), "-o",
+                    str(tmp_path / "b")], check=True, capture_output=True)
+    n = 20000
+    r = np.random.default_rng(5)
+    P = np.tile(NITINOL, (n, 1))
+    P[:, 0] = 10.0 ** r.uniform(2, 12, n)
+    P[:, 1] = r.choice([-0.5, 0.0, 0.33, 0.4999, 0.4999999], n)
+    P[:, 2] = r.choice([0.0, 0.01, 0.05], n)
+    size = 10.0 ** r.uniform(-17, -4, n)
+    G2 = P[:, 0] / (1 + P[:, 1])
+    P[:, [3, 4, 9, 10]] = (G2 * size)[:, None] * 10.0 ** r.uniform(-3, 9, (n, 1)) * r.uniform(0.5, 2.0, (n, 4))
+    P[::17, 3] = 0.0
+    P[::19, 3] *= -1.0
+    F = np.eye(3) + size[:, None, None] * r.normal(size=(n, 3, 3))
+    F[::7] = np.eye(3)
+    q, _ = np.linalg.qr(r.normal(size=(n, 3, 3)))
+    F[::5] = F[::5] @ q[::5]
+    xs = r.choice([0.0, 0.0, 0.0, -0.0, 1e-300, 0.5, np.nan], n)
+    f = np.where(r.uniform(size=n) < 0.7, 0.0, G2 * size * r.normal(size=n))
+    f[::23] = np.nan
+    b = np.concatenate([P, F.transpose(0, 2, 1).reshape(-1, 9), np.stack([xs, f, f], 1)], 1)
+    o = subprocess.run([str(tmp_path / "b")], input=np.ascontiguousarray(b).tobytes(), capture_output=True, check=True)
+    a, s = np.frombuffer(o.stdout).reshape(-1, 2, 10).transpose(1, 0, 2)
+    np.testing.assert_array_equal(a[:, 3], s[:, 3])
+    # the stress of points with martensite or an active branch: tests/test_law_paths.py
+    idle = ((s[:, 3].astype(int) & 3) == 0) & (s[:, 0] == 0.0)
+    a, s, P, G2 = a[idle], s[idle], P[idle], G2[idle]
+    np.testing.assert_array_equal(a[:, 0], s[:, 0])
+    K = np.abs(P[:, 0] / (3 * (1 - 2 * P[:, 1])))
+    s3 = np.sqrt(1 / 3)
+    with np.errstate(invalid="ignore"):
+        alfa = np.abs(np.sqrt(2 / 3) * (P[:, 4] - P[:, 3]) / (P[:, 4] + P[:, 3]) * s3) + s3
+    tol = 64 * 2.0 ** -52 * (G2 + 3 * K + 9 * np.nan_to_num(alfa, nan=1.0, posinf=1.0) * K)
+    d = np.abs(a[:, 4:] - s[:, 4:]).max(1)
+    same = (a == s) | (np.isnan(a) & np.isnan(s))
+    assert (same[:, 4:].all(1) | (d <= tol)).all()
+    assert (same[:, 1:3].all(1) | (np.abs(a[:, 1:3] - s[:, 1:3]).max(1) <= tol)).all()
